@@ -46,17 +46,23 @@ struct Geom {
     int px, gy, gz;
     long long nvol;      // elements per plane
     double dx, dy, dz;
+    double hdx;          // dx / 2
+    double ds[3];        // face areas dy dz, dx dz, dx dy
     double xmin, xmax, ymin, ymax, zmin, zmax;
     __host__ __device__ __forceinline__ long long idx(int i, int j, int k) const
     {
         return (long long)(i + 2) + (long long)px * ((long long)(j + 2) + (long long)gy * (k + 2));
     }
-    __device__ __forceinline__ double xc(int i) const { return xmin + dx / 2 + (double)(i - 1) * dx; }
+    __device__ __forceinline__ double xc(int i) const { return xmin + hdx + (double)(i - 1) * dx; }
 };
 
 struct Phys {
     double gamma, ciso, omega0, courant;
     double nu, eta;
+    // formed on the host: there are no scalar float64 instructions, so every
+    // thread of a kernel would hold these in vector registers
+    double smallp;       // pressure floor, commons.f90:52
+    double entho;        // 1 / (gamma - 1), gamma in the bulk type
     int iso, slope_type, riemann, riemann2d, fargo;
     int bc[3];
 };

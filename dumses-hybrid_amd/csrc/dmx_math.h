@@ -32,10 +32,12 @@ template <typename T> __device__ __forceinline__ T fab(T x) { return fabs(x); }
 template <typename T>
 __device__ __forceinline__ T tvd_slope(T qm1, T q0, T qp1, int st)
 {
-    const T s = T(st);
+    // st is 1 or 2: the division by st is an exact multiplication, where a
+    // division by a run-time value would take 11 instructions in float64
+    const T s = T(st), rs = st == 1 ? K<T>::one : K<T>::half;
     T dlft = s * (q0 - qm1);
     T drgt = s * (qp1 - q0);
-    T dcen = K<T>::half * (dlft + drgt) / s;
+    T dcen = K<T>::half * (dlft + drgt) * rs;
     T dsgn = sgn1(dcen);
     T slop = fmn(fab(dlft), fab(drgt));
     T dlim = slop;
@@ -57,7 +59,8 @@ __device__ __forceinline__ T cfast_b2(T gamma, T ploc, T r, T bn, T b2)
 // ---------------------------------------------------------------------------
 // 1D Riemann solvers, solver.f90:393-935.
 // q = [r, p, u_n, B_n, u_t1, B_t1, u_t2, B_t2]; fg[8]; pstar = total pressure
-// of the sampled state (HLLD only; 0 for the others, as pgstar is zeroed).
+// of the sampled state (HLLD only; 0 for the others, as pgstar is zeroed);
+// entho = 1 / (gamma - 1).
 //
 // The energy chain -- total energies and pressures, v.B, the star-state
 // energies, the energy flux, and the total-pressure differences that set
@@ -97,13 +100,12 @@ __device__ __forceinline__ void phys_flux(T r, T ploc, T u, T v, T w, T a, T b, 
 
 // hlld, solver.f90:618-836
 template <typename T>
-__device__ __forceinline__ void hlld1d(const T* ql, const T* qr, T gamma, T ploc, T proc,
+__device__ __forceinline__ void hlld1d(const T* ql, const T* qr, T gamma, D entho, T ploc, T proc,
                                        T* fg, T& pstar)
 {
     const T zero = K<T>::zero, half = K<T>::half;
     T rl = ql[0], ul = ql[2], al = ql[3], vl = ql[4], bl = ql[5], wl = ql[6], cl = ql[7];
     T rr = qr[0], ur = qr[2], ar = qr[3], vr = qr[4], br = qr[5], wr = qr[6], cr = qr[7];
-    const D entho = 1.0 / (D(gamma) - 1.0);
     T a = half * (al + ar);
     T sgnm = sgn1(a);
     D ecinl = 0.5 * ((D(ul) * ul + D(vl) * vl) + D(wl) * wl) * rl;
@@ -200,12 +202,11 @@ __device__ __forceinline__ void hlld1d(const T* ql, const T* qr, T gamma, T ploc
 
 // llf (solver.f90:393-498), hll (:504-612), upwind (:842-935)
 template <typename T, int SOLVER>
-__device__ __forceinline__ void simple1d(const T* ql, const T* qr, T gamma, T ploc, T proc, T* fg)
+__device__ __forceinline__ void simple1d(const T* ql, const T* qr, T gamma, D entho, T ploc, T proc, T* fg)
 {
     const T zero = K<T>::zero, half = K<T>::half;
     T rl = ql[0], ul = ql[2], al = ql[3], vl = ql[4], bl = ql[5], wl = ql[6], cl = ql[7];
     T rr = qr[0], ur = qr[2], ar = qr[3], vr = qr[4], br = qr[5], wr = qr[6], cr = qr[7];
-    const D entho = 1.0 / (D(gamma) - 1.0);
     T a = half * (al + ar);
     T fl[8], cL[8], fr[8], cR[8];
     D flE, cLE, frE, cRE;
@@ -235,15 +236,15 @@ __device__ __forceinline__ void simple1d(const T* ql, const T* qr, T gamma, T pl
 }
 
 template <typename T, int SOLVER>
-__device__ __forceinline__ void riemann1d(const T* ql, const T* qr, T gamma, T c2iso, bool iso,
+__device__ __forceinline__ void riemann1d(const T* ql, const T* qr, T gamma, D entho, T c2iso, bool iso,
                                           T* fg, T& pstar)
 {
     T ploc = iso ? ql[0] * c2iso : ql[1];
     T proc = iso ? qr[0] * c2iso : qr[1];
     if (SOLVER == 4) {
-        hlld1d(ql, qr, gamma, ploc, proc, fg, pstar);
+        hlld1d(ql, qr, gamma, entho, ploc, proc, fg, pstar);
     } else {
-        simple1d<T, SOLVER>(ql, qr, gamma, ploc, proc, fg);
+        simple1d<T, SOLVER>(ql, qr, gamma, entho, ploc, proc, fg);
         pstar = K<T>::zero;
     }
 }
@@ -424,6 +425,329 @@ __device__ __forceinline__ T riemann2d(const T* LL, const T* RL, const T* LR, co
            - ST * SB / (ST - SB) * (RR[4] - LL[4]))
           + SR * SL / (SR - SL) * (RR[5] - LL[5]);
     return e * dt;
+}
+
+// ---------------------------------------------------------------------------
+// float64 HLLD with shared reciprocals.
+//
+// An IEEE division of doubles is about 11 instructions here and a square root
+// about 18, most of them scaling for operands near the ends of the exponent
+// range, and the divisions by one denominator cannot share its reciprocal
+// because the scaling depends on both operands.  With operands known to lie
+// well inside the range the scaling is not needed: Newton's reciprocal (two
+// steps from v_rcp_f64), then one residual correction per quotient
+// (Markstein, IBM J. Res. Dev. 34, 1990), and Goldschmidt's square root with
+// two residual corrections (Markstein, RNC-6, 2004) round correctly, so the
+// bits are those of a / b and sqrt(x): 5 + 3 instructions per quotient,
+// 5 + 3 n for n quotients over one denominator, and 10 per square root.
+//
+// hlld1d_fast and hlld2d_fast evaluate hlld1d and hlld2d with them, in the
+// same order of operations, and return whether the operands were in range:
+// no NaN or infinity, no speed or root that vanishes, no numerator that is
+// tiny but not zero where its last bits could reach the result.  Otherwise
+// the caller evaluates hlld1d or hlld2d.  A maximum of square roots is the
+// root of the maximum (rounding is monotone), which removes the outer root
+// of all fast speeds but one per direction.  The face/edge kernel at 256^3
+// issues 4700 vector instructions a wave and plane instead of 6800 and takes
+// 4.88 ms instead of 5.50: it is left bound by its reads of the trace summary
+// (29 GB at 6.5 TB/s), 51% of its cycles issue vector instructions, 61%
+// before.  At 32 x 64 x 32 it takes 0.047 ms instead of 0.055.
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ double rcp_nr(double b)
+{
+    double y = __builtin_amdgcn_rcp(b);
+    double e = __builtin_fma(-b, y, 1.0);
+    y = __builtin_fma(y, e, y);
+    e = __builtin_fma(-b, y, 1.0);
+    return __builtin_fma(y, e, y);
+}
+// a / b with y = rcp_nr(b); the sign of a zero quotient is lost when a is -0
+__device__ __forceinline__ double div_nr(double a, double b, double y)
+{
+    const double q = a * y;
+    return __builtin_fma(__builtin_fma(-b, q, a), y, q);
+}
+// the same with the sign of a zero quotient
+__device__ __forceinline__ double div_nr0(double a, double b, double y)
+{
+    return __builtin_amdgcn_div_fixup(div_nr(a, b, y), b, a);
+}
+// 1 / b
+__device__ __forceinline__ double inv_nr(double b)
+{
+    const double y = rcp_nr(b);
+    return __builtin_fma(__builtin_fma(-b, y, 1.0), y, y);
+}
+// sqrt(x), x > 0
+__device__ __forceinline__ double sqrt_nr(double x)
+{
+    const double y = __builtin_amdgcn_rsq(x);
+    double g = x * y, h = 0.5 * y;
+    const double r = __builtin_fma(-h, g, 0.5);
+    g = __builtin_fma(g, r, g);
+    h = __builtin_fma(h, r, h);
+    g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
+    return __builtin_fma(__builtin_fma(-g, g, x), h, g);
+}
+// x is not zero but smaller than lim
+__device__ __forceinline__ bool tiny(double x, double lim) { return __builtin_fabs(x) < lim && x != 0.0; }
+
+// limits of the operand range: sums of densities, energies, pressures and
+// speeds below 2^100; distances of the outer waves from the contact above
+// 2^-100; discriminants of the fast speeds above 2^-500; numerators zero or
+// above 2^-700, except where the quotient is lost in the sum it enters.
+// Densities are at least 1e-10 (smallr).  With these every denominator lies
+// in 2^+-400, every root's argument in 2^+-700, and every residual is exact.
+constexpr double kHuge = 0x1p100, kGap = 0x1p-100, kDisc = 0x1p-500, kNum = 0x1p-700;
+
+__device__ __forceinline__ bool hlld1d_fast(const double* ql, const double* qr, double gamma, double entho, double ploc,
+                                            double proc, double* fg, double& pstar)
+{
+    const double zero = 0.0, half = 0.5;
+    double rl = ql[0], ul = ql[2], al = ql[3], vl = ql[4], bl = ql[5], wl = ql[6], cl = ql[7];
+    double rr = qr[0], ur = qr[2], ar = qr[3], vr = qr[4], br = qr[5], wr = qr[6], cr = qr[7];
+    double a = half * (al + ar);
+    double sgnm = sgn1(a);
+    double ecinl = 0.5 * ((ul * ul + vl * vl) + wl * wl) * rl;
+    double emagl = 0.5 * ((a * a + bl * bl) + cl * cl);
+    double etotl = (ploc * entho + ecinl) + emagl;
+    double ptotl = ploc + emagl;
+    double vdotbl = (ul * a + vl * bl) + wl * cl;
+    double ecinr = 0.5 * ((ur * ur + vr * vr) + wr * wr) * rr;
+    double emagr = 0.5 * ((a * a + br * br) + cr * cr);
+    double etotr = (proc * entho + ecinr) + emagr;
+    double ptotr = proc + emagr;
+    double vdotbr = (ur * a + vr * br) + wr * cr;
+    // discriminant and half sum of the fast speed (cfast_b2)
+    auto speed = [&](double p, double r, double b2, double& d2) {
+        const double y = rcp_nr(r);
+        const double c2 = div_nr(gamma * p, r, y);
+        d2 = half * (c2 + div_nr(b2, r, y));
+        return d2 * d2 - div_nr(c2 * a * a, r, y);
+    };
+    double d2l, d2r;
+    const double discl = speed(ploc, rl, (a * a + bl * bl) + cl * cl, d2l);
+    const double discr = speed(proc, rr, (a * a + br * br) + cr * cr, d2r);
+    const double cf = sqrt_nr(__builtin_fmax(d2l + sqrt_nr(discl), d2r + sqrt_nr(discr)));
+    const double umin = __builtin_fmin(ul, ur), umax = __builtin_fmax(ul, ur);
+    const double sl = umin - cf, sr = umax + cf;
+    double rcl = rl * (ul - sl);
+    double rcr = rr * (sr - ur);
+    const double den = rcr + rcl, yden = rcp_nr(den);
+    const double nus = (rcr * ur + rcl * ul) + (ptotl - ptotr);
+    const double ustar = div_nr(nus, den, yden);
+    const double ptotstar = div_nr((rcr * ptotl + rcl * ptotr) + rcl * rcr * (ul - ur), den, yden);
+    const double dl = sl - ustar, dr = sr - ustar;
+    bool ok = __builtin_fmin(discl, discr) > kDisc && sl < umin && sr > umax && dl < -kGap && dr > kGap
+              && ((etotl + etotr) + (rl + rr)) + ((sr - sl) + den) < kHuge && !tiny(nus, kNum);
+    // n / d with y = rcp_nr(d), and v - n / d, where v may absorb a tiny quotient
+    auto quot = [&](double n, double d, double y) {
+        ok = ok && !tiny(n, kNum);
+        return div_nr0(n, d, y);
+    };
+    auto less_quot = [&](double v, double n, double d, double y) {
+        const double q = div_nr0(n, d, y);
+        ok = ok && !(tiny(n, kNum) && !(fab(q) < 0x1p-60 * fab(v)));
+        return v - q;
+    };
+    auto star = [&](double r, double u, double v, double w, double b, double c, double s, double ds, double etot,
+                    double ptot, double vdotb, double& rstar, double& vstar, double& bstar, double& wstar,
+                    double& cstar, double& vdotbstar, double& etotstar) {
+        const double yd = rcp_nr(ds);
+        rstar = div_nr(r * (s - u), ds, yd);
+        const double estar = r * (s - u) * ds - a * a;
+        const double e = r * (s - u) * (s - u) - a * a;
+        ok = ok && estar != zero;
+        const double ye = rcp_nr(estar);
+        vstar = less_quot(v, a * b * (ustar - u), estar, ye);
+        bstar = quot(b * e, estar, ye);
+        wstar = less_quot(w, a * c * (ustar - u), estar, ye);
+        cstar = quot(c * e, estar, ye);
+        vdotbstar = (ustar * a + vstar * bstar) + wstar * cstar;
+        etotstar = div_nr((((s - u) * etot - ptot * u) + ptotstar * ustar) + a * (vdotb - vdotbstar), ds, yd);
+    };
+    double rstarl, vstarl, bstarl, wstarl, cstarl, vdotbstarl, etotstarl;
+    double rstarr, vstarr, bstarr, wstarr, cstarr, vdotbstarr, etotstarr;
+    star(rl, ul, vl, wl, bl, cl, sl, dl, etotl, ptotl, vdotbl, rstarl, vstarl, bstarl, wstarl, cstarl, vdotbstarl,
+         etotstarl);
+    star(rr, ur, vr, wr, br, cr, sr, dr, etotr, ptotr, vdotbr, rstarr, vstarr, bstarr, wstarr, cstarr, vdotbstarr,
+         etotstarr);
+    const double sqrrstarl = sqrt_nr(rstarl), sqrrstarr = sqrt_nr(rstarr);
+    const double sal = ustar - div_nr(fab(a), sqrrstarl, rcp_nr(sqrrstarl));
+    const double sar = ustar + div_nr(fab(a), sqrrstarr, rcp_nr(sqrrstarr));
+    const double dens = sqrrstarl + sqrrstarr, ys = rcp_nr(dens);
+    const double vss = quot((sqrrstarl * vstarl + sqrrstarr * vstarr) + sgnm * (bstarr - bstarl), dens, ys);
+    const double wss = quot((sqrrstarl * wstarl + sqrrstarr * wstarr) + sgnm * (cstarr - cstarl), dens, ys);
+    const double bss = quot((sqrrstarl * bstarr + sqrrstarr * bstarl) + sgnm * sqrrstarl * sqrrstarr * (vstarr - vstarl),
+                            dens, ys);
+    const double css = quot((sqrrstarl * cstarr + sqrrstarr * cstarl) + sgnm * sqrrstarl * sqrrstarr * (wstarr - wstarl),
+                            dens, ys);
+    const double vdotbss = (ustar * a + vss * bss) + wss * css;
+    const double etotssl = etotstarl - sgnm * sqrrstarl * (vdotbstarl - vdotbss);
+    const double etotssr = etotstarr + sgnm * sqrrstarr * (vdotbstarr - vdotbss);
+    // the sampled state: outer (0), star (1) or double star (2), left or right
+    double ro, uo, vo, wo, bo, co, ptoto, etoto, vdotbo;
+    if (sl > zero) {
+        ro = rl; uo = ul; vo = vl; wo = wl; bo = bl; co = cl; ptoto = ptotl; etoto = etotl; vdotbo = vdotbl;
+    } else if (sal > zero) {
+        ro = rstarl; uo = ustar; vo = vstarl; wo = wstarl; bo = bstarl; co = cstarl; ptoto = ptotstar;
+        etoto = etotstarl; vdotbo = vdotbstarl;
+    } else if (ustar > zero) {
+        ro = rstarl; uo = ustar; vo = vss; wo = wss; bo = bss; co = css; ptoto = ptotstar;
+        etoto = etotssl; vdotbo = vdotbss;
+    } else if (sar > zero) {
+        ro = rstarr; uo = ustar; vo = vss; wo = wss; bo = bss; co = css; ptoto = ptotstar;
+        etoto = etotssr; vdotbo = vdotbss;
+    } else if (sr > zero) {
+        ro = rstarr; uo = ustar; vo = vstarr; wo = wstarr; bo = bstarr; co = cstarr; ptoto = ptotstar;
+        etoto = etotstarr; vdotbo = vdotbstarr;
+    } else {
+        ro = rr; uo = ur; vo = vr; wo = wr; bo = br; co = cr; ptoto = ptotr; etoto = etotr; vdotbo = vdotbr;
+    }
+    fg[0] = ro * uo;
+    fg[1] = (etoto + ptoto) * uo - a * vdotbo;
+    fg[2] = ro * uo * uo - a * a;
+    fg[3] = zero;
+    fg[4] = ro * uo * vo - a * bo;
+    fg[5] = bo * uo - a * vo;
+    fg[6] = ro * uo * wo - a * co;
+    fg[7] = co * uo - a * wo;
+    pstar = ptoto;
+    return ok;
+}
+
+__device__ __forceinline__ bool hlld2d_fast(const double* LL, const double* RL, const double* LR, const double* RR,
+                                            double dt, double gamma, double& emf)
+{
+    const double zero = 0.0, half = 0.5, smallc = 1e-10;
+    double rLL = LL[0], pLL = LL[1], uLL = LL[2], vLL = LL[3], ALL = LL[4], BLL = LL[5], CLL = LL[6], ELL = LL[7];
+    double rRL = RL[0], pRL = RL[1], uRL = RL[2], vRL = RL[3], ARL = RL[4], BRL = RL[5], CRL = RL[6], ERL = RL[7];
+    double rLR = LR[0], pLR = LR[1], uLR = LR[2], vLR = LR[3], ALR = LR[4], BLR = LR[5], CLR = LR[6], ELR = LR[7];
+    double rRR = RR[0], pRR = RR[1], uRR = RR[2], vRR = RR[3], ARR = RR[4], BRR = RR[5], CRR = RR[6], ERR = RR[7];
+#define MX4(a, b, c, d) __builtin_fmax(__builtin_fmax(__builtin_fmax(a, b), c), d)
+#define MN4(a, b, c, d) __builtin_fmin(__builtin_fmin(__builtin_fmin(a, b), c), d)
+    // squared fast speeds along both directions, the least discriminant
+    double cx2 = zero, cy2 = zero, disc = kHuge;
+    auto speeds = [&](const double* q) {
+        const double y = rcp_nr(q[0]);
+        const double c2 = div_nr(gamma * q[1], q[0], y);
+        const double d2 = half * (c2 + div_nr((q[4] * q[4] + q[5] * q[5]) + q[6] * q[6], q[0], y));
+        const double x = d2 * d2 - div_nr(c2 * q[4] * q[4], q[0], y);
+        const double z = d2 * d2 - div_nr(c2 * q[5] * q[5], q[0], y);
+        disc = __builtin_fmin(disc, __builtin_fmin(x, z));
+        cx2 = __builtin_fmax(cx2, d2 + sqrt_nr(x));
+        cy2 = __builtin_fmax(cy2, d2 + sqrt_nr(z));
+    };
+    speeds(LL);
+    speeds(LR);
+    speeds(RL);
+    speeds(RR);
+    const double cx = sqrt_nr(cx2), cy = sqrt_nr(cy2);
+    const double umin = MN4(uLL, uLR, uRL, uRR), umax = MX4(uLL, uLR, uRL, uRR);
+    const double vmin = MN4(vLL, vLR, vRL, vRR), vmax = MX4(vLL, vLR, vRL, vRR);
+    double SL = umin - cx, SR = umax + cx, SB = vmin - cy, ST = vmax + cy;
+    double PtotLL = pLL + 0.5 * ((ALL * ALL + BLL * BLL) + CLL * CLL);
+    double PtotLR = pLR + 0.5 * ((ALR * ALR + BLR * BLR) + CLR * CLR);
+    double PtotRL = pRL + 0.5 * ((ARL * ARL + BRL * BRL) + CRL * CRL);
+    double PtotRR = pRR + 0.5 * ((ARR * ARR + BRR * BRR) + CRR * CRR);
+    double rcLLx = rLL * (uLL - SL), rcRLx = rRL * (SR - uRL);
+    double rcLRx = rLR * (uLR - SL), rcRRx = rRR * (SR - uRR);
+    double rcLLy = rLL * (vLL - SB), rcLRy = rLR * (ST - vLR);
+    double rcRLy = rRL * (vRL - SB), rcRRy = rRR * (ST - vRR);
+    const double nus = (((rcLLx * uLL + rcLRx * uLR) + rcRLx * uRL) + rcRRx * uRR)
+                       + (((PtotLL - PtotRL) + PtotLR) - PtotRR);
+    const double nvs = (((rcLLy * vLL + rcLRy * vLR) + rcRLy * vRL) + rcRRy * vRR)
+                       + (((PtotLL - PtotLR) + PtotRL) - PtotRR);
+    const double dus = ((rcLLx + rcLRx) + rcRLx) + rcRRx, dvs = ((rcLLy + rcLRy) + rcRLy) + rcRRy;
+    const double ustar = div_nr(nus, dus, rcp_nr(dus)), vstar = div_nr(nvs, dvs, rcp_nr(dvs));
+    const double dSL = SL - ustar, dSR = SR - ustar, dSB = SB - vstar, dST = ST - vstar;
+    const bool ok = disc > kDisc && SL < umin && SR > umax && SB < vmin && ST > vmax && dSL < -kGap && dSR > kGap
+                    && dSB < -kGap && dST > kGap && !tiny(nus, kNum) && !tiny(nvs, kNum)
+                    && (((PtotLL + PtotLR) + (PtotRL + PtotRR)) + ((rLL + rLR) + (rRL + rRR)))
+                               + (((SR - SL) + (ST - SB)) + (dus + dvs))
+                           < kHuge;
+    double SLustar = inv_nr(dSL), SRustar = inv_nr(dSR);
+    double SBvstar = inv_nr(dSB), STvstar = inv_nr(dST);
+
+    double rstarLLx = rLL * (SL - uLL) * SLustar, BstarLL = BLL * (SL - uLL) * SLustar;
+    double rstarLLy = rLL * (SB - vLL) * SBvstar, AstarLL = ALL * (SB - vLL) * SBvstar;
+    double rstarLL = rLL * (SL - uLL) * SLustar * (SB - vLL) * SBvstar;
+    double EstarLLx = ustar * BstarLL - vLL * ALL, EstarLLy = uLL * BLL - vstar * AstarLL;
+    double EstarLL = ustar * BstarLL - vstar * AstarLL;
+
+    double rstarLRx = rLR * (SL - uLR) * SLustar, BstarLR = BLR * (SL - uLR) * SLustar;
+    double rstarLRy = rLR * (ST - vLR) * STvstar, AstarLR = ALR * (ST - vLR) * STvstar;
+    double rstarLR = rLR * (SL - uLR) * SLustar * (ST - vLR) * STvstar;
+    double EstarLRx = ustar * BstarLR - vLR * ALR, EstarLRy = uLR * BLR - vstar * AstarLR;
+    double EstarLR = ustar * BstarLR - vstar * AstarLR;
+
+    double rstarRLx = rRL * (SR - uRL) * SRustar, BstarRL = BRL * (SR - uRL) * SRustar;
+    double rstarRLy = rRL * (SB - vRL) * SBvstar, AstarRL = ARL * (SB - vRL) * SBvstar;
+    double rstarRL = rRL * (SR - uRL) * SRustar * (SB - vRL) * SBvstar;
+    double EstarRLx = ustar * BstarRL - vRL * ARL, EstarRLy = uRL * BRL - vstar * AstarRL;
+    double EstarRL = ustar * BstarRL - vstar * AstarRL;
+
+    double rstarRRx = rRR * (SR - uRR) * SRustar, BstarRR = BRR * (SR - uRR) * SRustar;
+    double rstarRRy = rRR * (ST - vRR) * STvstar, AstarRR = ARR * (ST - vRR) * STvstar;
+    double rstarRR = rRR * (SR - uRR) * SRustar * (ST - vRR) * STvstar;
+    double EstarRRx = ustar * BstarRR - vRR * ARR, EstarRRy = uRR * BRR - vstar * AstarRR;
+    double EstarRR = ustar * BstarRR - vstar * AstarRR;
+
+    // Alfven speeds |field| / sqrt(density)
+    auto alf = [](double b, double r) {
+        const double s = sqrt_nr(r);
+        return div_nr(fab(b), s, rcp_nr(s));
+    };
+    const double sqLR = inv_nr(sqrt_nr(rstarLR)), sqRL = inv_nr(sqrt_nr(rstarRL));
+    const double sqRR = inv_nr(sqrt_nr(rstarRR)), sqLL = inv_nr(sqrt_nr(rstarLL));
+    const double calfvenL = __builtin_fmax(
+        MX4(alf(ALR, rstarLRx), fab(AstarLR) * sqLR, alf(ALL, rstarLLx), fab(AstarLL) * sqLL), smallc);
+    const double calfvenR = __builtin_fmax(
+        MX4(alf(ARR, rstarRRx), fab(AstarRR) * sqRR, alf(ARL, rstarRLx), fab(AstarRL) * sqRL), smallc);
+    const double calfvenB = __builtin_fmax(
+        MX4(alf(BLL, rstarLLy), fab(BstarLL) * sqLL, alf(BRL, rstarRLy), fab(BstarRL) * sqRL), smallc);
+    const double calfvenT = __builtin_fmax(
+        MX4(alf(BLR, rstarLRy), fab(BstarLR) * sqLR, alf(BRR, rstarRRy), fab(BstarRR) * sqRR), smallc);
+#undef MX4
+#undef MN4
+    const double SAL = __builtin_fmin(ustar - calfvenL, zero), SAR = __builtin_fmax(ustar + calfvenR, zero);
+    const double SAB = __builtin_fmin(vstar - calfvenB, zero), SAT = __builtin_fmax(vstar + calfvenT, zero);
+    const double SARSAL = inv_nr(SAR - SAL);
+    const double SATSAB = inv_nr(SAT - SAB);
+    double AstarT = (SAR * AstarRR - SAL * AstarLR) * SARSAL;
+    double AstarB = (SAR * AstarRL - SAL * AstarLL) * SARSAL;
+    double BstarR = (SAT * BstarRR - SAB * BstarRL) * SATSAB;
+    double BstarL = (SAT * BstarLR - SAB * BstarLL) * SATSAB;
+    double E;
+    if (SB > zero) {
+        if (SL > zero) E = ELL;
+        else if (SR < zero) E = ERL;
+        else E = ((SAR * EstarLLx - SAL * EstarRLx) + SAR * SAL * (BRL - BLL)) * SARSAL;
+    } else if (ST < zero) {
+        if (SL > zero) E = ELR;
+        else if (SR < zero) E = ERR;
+        else E = ((SAR * EstarLRx - SAL * EstarRRx) + SAR * SAL * (BRR - BLR)) * SARSAL;
+    } else if (SL > zero) {
+        E = ((SAT * EstarLLy - SAB * EstarLRy) - SAT * SAB * (ALR - ALL)) * SATSAB;
+    } else if (SR < zero) {
+        E = ((SAT * EstarRLy - SAB * EstarRRy) - SAT * SAB * (ARR - ARL)) * SATSAB;
+    } else {
+        E = (((((SAL * SAB * EstarRR - SAL * SAT * EstarRL) - SAR * SAB * EstarLR) + SAR * SAT * EstarLL) * SARSAL) * SATSAB
+             - SAT * SAB * SATSAB * (AstarT - AstarB))
+            + SAR * SAL * SARSAL * (BstarR - BstarL);
+    }
+    emf = E * dt;
+    return ok;
+}
+
+// float bulk takes the hardware's approximate division and root already
+__device__ __forceinline__ bool hlld1d_fast(const float*, const float*, float, double, float, float, float*, float&)
+{
+    return false;
+}
+__device__ __forceinline__ bool hlld2d_fast(const float*, const float*, const float*, const float*, float, float, float&)
+{
+    return false;
 }
 
 } // namespace dmx
