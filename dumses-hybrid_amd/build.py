@@ -25,6 +25,7 @@ COMMON = ["-O3", "-fPIC", "-std=c++17", f"--offload-arch={ARCH}",
 UNITS = [
     ("dmx_f64.hip", ["-ffp-contract=off"]),
     ("dmx_f32.hip", ["-ffp-contract=fast", "-ffast-math", "-fno-finite-math-only"]),
+    ("dmx_f32l.hip", ["-ffp-contract=fast", "-ffast-math", "-fno-finite-math-only"]),
     ("dmx_abi.cpp", []),
     ("dmx_mlp.hip", ["-ffp-contract=fast"]),
 ]

@@ -96,7 +96,9 @@ int dmx_create(const dmx_params* p, dmx_ctx** ctx)
         dmx::set_error("no HIP device");
         return DMX_E_HIP;
     }
-    dmx::Engine* e = p->precision == DMX_FP32 ? dmx::make_engine_f32(*p, &rc) : dmx::make_engine_f64(*p, &rc);
+    dmx::Engine* e = p->precision != DMX_FP32 ? dmx::make_engine_f64(*p, &rc)
+                     : p->slope_type == 4     ? dmx::make_engine_f32l(*p, &rc)
+                                              : dmx::make_engine_f32(*p, &rc);
     if (!e) return rc ? rc : DMX_E_HIP;
     *ctx = new dmx_ctx{e, *p};
     return DMX_OK;

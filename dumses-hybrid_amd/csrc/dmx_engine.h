@@ -1,9 +1,10 @@
 // dmx_engine.h -- host-side engine interface behind the C ABI.
 //
 // One Engine owns one device-resident domain and one HIP stream.  The float64
-// and float32 engines are built from the same kernel source in two
-// translation units (dmx_f64.hip, dmx_f32.hip); dmx_abi.cpp picks one per
-// context from dmx_params.precision.
+// and float32 engines are built from the same kernel source in three
+// translation units (dmx_f64.hip, dmx_f32.hip, and dmx_f32l.hip for float32
+// with the learned limiter); dmx_abi.cpp picks one per context from
+// dmx_params.precision and slope_type.
 #pragma once
 
 #include <stdint.h>
@@ -30,6 +31,9 @@ public:
     virtual int set_shape(const int* shape) = 0;
     virtual int set_limiter(const float* theta, int n) = 0;
     virtual int learned_slopes(float* out, double* fallback) = 0;
+    // 0: float64, 1: float32, 2: float32 with the learned limiter
+    virtual int kind() const = 0;
+    virtual bool uploaded() const = 0;
 };
 
 // Several contexts of one precision advanced together (dmx_batch_*): every
@@ -54,6 +58,7 @@ void set_error(const char* fmt, ...);
 
 Engine* make_engine_f64(const dmx_params& p, int* rc);
 Engine* make_engine_f32(const dmx_params& p, int* rc);
+Engine* make_engine_f32l(const dmx_params& p, int* rc);
 Batch* make_batch_f64(Engine* const* es, int n, int nstreams, int* rc);
 Batch* make_batch_f32(Engine* const* es, int n, int nstreams, int* rc);
 // dmx_compute_dt_noalloc (float64 state in the caller's device memory;

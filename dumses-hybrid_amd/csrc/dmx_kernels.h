@@ -10,7 +10,7 @@
 //        from it; B: the CT face-B accumulation stays float64 in both
 //        precisions).  The reference's right faces are implied:
 //        B_R(i) = B_L(i+1).
-//   S  : 47 values of T per cell, the per-cell trace summary written by the
+//   S  : 38 (47) values of T per cell, the per-cell trace summary written by the
 //        trace kernel for cells [0, n+1]^3 (see TraceSlot), in groups of
 //        256 bytes of consecutive cells per slot (s_off in dmx_step.inc).
 //   F  : 18 planes of T, x/y/z face fluxes of rho, rho*u, rho*v, rho*w, E
@@ -24,6 +24,17 @@
 
 #include "dmx_tiling.h"
 
+// 1: the trace summary holds the fields of both faces of a cell in each
+// direction (47 words) and the states at a face or edge take the mean of the
+// two cells' values.  float32 contexts with the learned limiter are built so
+// (dmx_f32l.hip): the two values differ by a rounding there, and the limiter's
+// branches amplify the last bit of the state (1e-7 to 6e-5 within 30 steps at
+// 128^3), so its runs keep the arithmetic they had.  In float64 both forms
+// give the same bits.
+#ifndef DMX_BOTH_FACES
+#define DMX_BOTH_FACES 0
+#endif
+
 namespace dmx {
 
 enum TraceSlot {
@@ -31,11 +42,23 @@ enum TraceSlot {
     S_DRX = 8, S_DUX, S_DVX, S_DWX, S_DPX, S_DBX, S_DCX, // half slopes along x
     S_DRY = 15, S_DUY, S_DVY, S_DWY, S_DPY, S_DAY, S_DCY,
     S_DRZ = 22, S_DUZ, S_DVZ, S_DWZ, S_DPZ, S_DAZ, S_DBZ,
+#if DMX_BOTH_FACES
     S_AL = 29, S_AR, S_BL, S_BR, S_CL, S_CR,             // predicted face fields
     S_DALY = 35, S_DARY, S_DALZ, S_DARZ,                 // face-field half slopes
     S_DBLX, S_DBRX, S_DBLZ, S_DBRZ,
     S_DCLX, S_DCRX, S_DCLY, S_DCRY,
     NSLOT = 47
+#else
+    // predicted left face fields and their transverse half slopes: the right
+    // face of a cell is the left one of the next cell, whose predictor forms
+    // the same expressions.  Without the right faces a cell has 38 words, not
+    // 47: at 256^3 the float64 trace takes 1.79 ms (2.13), the face/edge
+    // stage 4.42 (4.88), both bound by the summary's traffic, and the float32
+    // fused kernel 2.67 (2.83), whose LDS tile is that much smaller
+    S_AL = 29, S_BL, S_CL,
+    S_DALY = 32, S_DALZ, S_DBLX, S_DBLZ, S_DCLX, S_DCLY,
+    NSLOT = 38
+#endif
 };
 
 // flux planes: F[d*6 + c], c in {rho, mx, my, mz, E, pstar}
