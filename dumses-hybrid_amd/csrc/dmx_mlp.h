@@ -23,19 +23,14 @@ constexpr int OFF_W1 = 0, OFF_B1 = OFF_W1 + NIN * NH, OFF_W2 = OFF_B1 + NH, OFF_
               OFF_W3 = OFF_B2 + NH, OFF_B3 = OFF_W3 + NH * NOUT, NPARAM = OFF_B3 + NOUT;
 static_assert(NPARAM == 7304, "parameter count");
 
-__device__ __forceinline__ float gelu(float x)
+// h = gelu(a) and d = gelu'(a)
+__device__ __forceinline__ void gelu_both(float a, float& h, float& d)
 {
     const float c = 0.7978845608028654f;   // sqrt(2/pi)
-    float t = tanhf(c * (x + 0.044715f * x * x * x));
-    return 0.5f * x * (1.0f + t);
-}
-
-__device__ __forceinline__ float gelu_grad(float x)
-{
-    const float c = 0.7978845608028654f;
-    float t = tanhf(c * (x + 0.044715f * x * x * x));
-    float du = c * (1.0f + 3.0f * 0.044715f * x * x);
-    return 0.5f * (1.0f + t) + 0.5f * x * (1.0f - t * t) * du;
+    const float t = tanhf(c * (a + 0.044715f * a * a * a));
+    const float du = c * (1.0f + 3.0f * 0.044715f * a * a);
+    h = 0.5f * a * (1.0f + t);
+    d = 0.5f * (1.0f + t) + 0.5f * a * (1.0f - t * t) * du;
 }
 
 // the 5 features of one variable and its scale

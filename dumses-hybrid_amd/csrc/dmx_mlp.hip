@@ -1,14 +1,14 @@
 // dmx_mlp.hip -- training of the learned slope limiter on the GPU:
 // forward and backward passes of the 40-64-64-8 GELU network (float32),
 // mean-squared-error loss, Adam, and on-device minibatch sampling from a
-// resident data set; plus a self-test of the bf16 MFMA lane layout that the
+// resident data set (two kernels a step); plus a self-test of the bf16 MFMA lane layout that the
 // inference kernel of the step relies on.
 #include <hip/hip_runtime.h>
 
 #include <stdint.h>
 #include <string.h>
 
-#include <vector>
+#include <algorithm>
 
 #include "dmx.h"
 #include "dmx_engine.h"
@@ -17,96 +17,8 @@
 namespace dmx {
 namespace mlp {
 
-// pre[s][o] = b[o] + sum_i in[s][i] W[i][o]; act = gelu(pre) when act != 0
-__global__ __launch_bounds__(256) void k_dense_fwd(const float* in, int nin, const float* W, const float* b,
-                                                   int nout, int n, float* pre, float* act)
-{
-    long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (long long)n * nout) return;
-    int s = (int)(t / nout), o = (int)(t % nout);
-    const float* x = in + (long long)s * nin;
-    float a = b[o];
-    for (int i = 0; i < nin; i++) a += x[i] * W[i * nout + o];
-    pre[t] = a;
-    if (act) act[t] = gelu(a);
-}
-
-// g = (y - T) / n and the per-block partial sums of 0.5 (y - T)^2 / n
-__global__ __launch_bounds__(256) void k_out_grad(const float* y, const float* T, int n, float* g, float* part)
-{
-    __shared__ float red[256];
-    long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    float l = 0.0f;
-    if (t < (long long)n * NOUT) {
-        float r = y[t] - T[t];
-        g[t] = r / (float)n;
-        l = 0.5f * r * r / (float)n;
-    }
-    red[threadIdx.x] = l;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) part[blockIdx.x] = red[0];
-}
-
-// gW[i][o] = sum_s in[s][i] g[s][o] (row i = nin gives the bias gradient):
-// one block per output column o, threads over (i, sample chunk)
-__global__ __launch_bounds__(256) void k_dense_wgrad(const float* in, int nin, const float* g, int nout, int n,
-                                                     float* gW, float* gb)
-{
-    __shared__ float red[256];
-    const int o = blockIdx.x;
-    for (int i = 0; i <= nin; i++) {
-        float a = 0.0f;
-        for (int s = threadIdx.x; s < n; s += 256) {
-            float x = i < nin ? in[(long long)s * nin + i] : 1.0f;
-            a += x * g[(long long)s * nout + o];
-        }
-        red[threadIdx.x] = a;
-        __syncthreads();
-        for (int w = 128; w > 0; w >>= 1) {
-            if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-            __syncthreads();
-        }
-        if (threadIdx.x == 0) {
-            if (i < nin) gW[i * nout + o] = red[0];
-            else gb[o] = red[0];
-        }
-        __syncthreads();
-    }
-}
-
-// gin[s][i] = gelu'(pre_in[s][i]) sum_o g[s][o] W[i][o]
-__global__ __launch_bounds__(256) void k_dense_igrad(const float* g, int nout, const float* W, int nin, int n,
-                                                     const float* pre_in, float* gin)
-{
-    long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (long long)n * nin) return;
-    int s = (int)(t / nin), i = (int)(t % nin);
-    const float* gs = g + (long long)s * nout;
-    float a = 0.0f;
-    for (int o = 0; o < nout; o++) a += gs[o] * W[i * nout + o];
-    gin[t] = a * gelu_grad(pre_in[t]);
-}
-
-// Adam (Kingma and Ba 2015), bias-corrected step size
-__global__ __launch_bounds__(256) void k_adam(float* th, const float* gr, float* m, float* v, int n, float lr,
-                                              float b1, float b2, float eps, float c1, float c2)
-{
-    int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n) return;
-    float g = gr[t];
-    float mm = b1 * m[t] + (1.0f - b1) * g;
-    float vv = b2 * v[t] + (1.0f - b2) * g * g;
-    m[t] = mm;
-    v[t] = vv;
-    th[t] -= lr * (mm / c1) / (sqrtf(vv / c2) + eps);
-}
-
-// minibatch of B rows drawn from n rows with a counter-based hash
-// (splitmix64 finaliser of seed + draw number)
+// minibatch of rows drawn from n rows with a counter-based hash (splitmix64
+// finaliser of seed + draw number)
 __device__ __forceinline__ unsigned long long mix64(unsigned long long z)
 {
     z = (z ^ (z >> 30)) * 0xbf58476d1ce4e5b9ULL;
@@ -114,14 +26,206 @@ __device__ __forceinline__ unsigned long long mix64(unsigned long long z)
     return z ^ (z >> 31);
 }
 
-__global__ __launch_bounds__(256) void k_gather(const float* X, const float* T, long long n, int B,
-                                                unsigned long long key, float* Xb, float* Tb)
+// ---------------------------------------------------------------------------
+// Forward and backward pass in one kernel.  A block takes tiles of TS rows
+// (tile blockIdx.x, + gridDim.x, ...) through the three layers with the
+// weights and every activation in LDS, and adds the tiles' parameter
+// gradients in registers; its sums go to part[block][NPARAM] and k_reduce
+// adds the blocks'.  With a launch per layer and pass the activations went
+// through HBM, and the weight gradients (one block per output column, a
+// reduction per weight) took most of a step: 0.90 ms a step of 4096 rows in
+// 11 launches, now 0.03 ms in 2.
+//
+// TS = 16 gives a batch of 4096 256 blocks, one per CU; larger batches give
+// a block several tiles.  W2 rows are padded to 65 words, so that the
+// backward pass reads its columns without bank conflicts.
+// ---------------------------------------------------------------------------
+constexpr int TS = 16, MAXBLK = 256, LW2S = NH + 1;
+
+struct TrainLds {
+    float w1[NIN * NH], w2[NH * LW2S], w3[NH * NOUT];
+    float b1[NH], b2[NH], b3[NOUT];
+    float x[NIN][TS], t[NOUT][TS];               // rows of the tile, transposed
+    float h1[NH][TS], d1[NH][TS];                // gelu(a1), gelu'(a1); then d1 holds dL/da1
+    float h2[NH][TS], d2[NH][TS];
+    float g3[NOUT][TS];                          // dL/dy
+    float loss[TS * NOUT];
+    long long row[TS];
+};
+
+// X, T: data (rows drawn by the hash of key when ndata > 0, else row s of the
+// batch is row s); n rows in the batch; y: outputs (may be null); part: block
+// gradients (null: forward only); lpart: block sums of 0.5 (y - T)^2 / n
+__global__ __launch_bounds__(256) void k_fwd_bwd(const float* __restrict__ X, const float* __restrict__ T, long long ndata,
+                                                 int n, unsigned long long key, const float* __restrict__ th,
+                                                 float* __restrict__ y, float* __restrict__ part,
+                                                 float* __restrict__ lpart)
 {
-    int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= B) return;
-    long long r = (long long)(mix64(key + (unsigned long long)b * 0x9e3779b97f4a7c15ULL) % (unsigned long long)n);
-    for (int i = 0; i < NIN; i++) Xb[(long long)b * NIN + i] = X[r * NIN + i];
-    for (int o = 0; o < NOUT; o++) Tb[(long long)b * NOUT + o] = T[r * NOUT + o];
+    __shared__ TrainLds L;
+    const int tid = threadIdx.x;
+    for (int i = tid; i < NIN * NH; i += 256) L.w1[i] = th[OFF_W1 + i];
+    for (int i = tid; i < NH * NH; i += 256) L.w2[(i / NH) * LW2S + i % NH] = th[OFF_W2 + i];
+    for (int i = tid; i < NH * NOUT; i += 256) L.w3[i] = th[OFF_W3 + i];
+    if (tid < NH) {
+        L.b1[tid] = th[OFF_B1 + tid];
+        L.b2[tid] = th[OFF_B2 + tid];
+    }
+    if (tid < NOUT) L.b3[tid] = th[OFF_B3 + tid];
+    // thread (o, q): column o of a layer, rows 4 q .. 4 q + 3 of the tile (and
+    // quarter q of a weight matrix's rows)
+    const int o = tid & 63, q = tid >> 6, s0 = 4 * q;
+    float gw1[NIN / 4] = {}, gw2[NH / 4] = {}, gw3[2] = {}, gb = 0.0f, lsum = 0.0f;
+    const float rows = (float)n;
+    const int ntile = (n + TS - 1) / TS;
+    for (int tile = blockIdx.x; tile < ntile; tile += gridDim.x) {
+        const int base = tile * TS;
+        __syncthreads();   // the previous tile's reads are done, the weights are there
+        if (tid < TS) {
+            const unsigned long long b = (unsigned long long)(base + tid);
+            L.row[tid] = ndata > 0 ? (long long)(mix64(key + b * 0x9e3779b97f4a7c15ULL) % (unsigned long long)ndata)
+                                   : (long long)b;
+        }
+        __syncthreads();
+        for (int e = tid; e < TS * NIN; e += 256) {
+            const int s = e / NIN, i = e - s * NIN;
+            L.x[i][s] = base + s < n ? X[L.row[s] * NIN + i] : 0.0f;
+        }
+        if (T && tid < TS * NOUT) {
+            const int s = tid / NOUT, i = tid % NOUT;
+            L.t[i][s] = base + s < n ? T[L.row[s] * NOUT + i] : 0.0f;
+        }
+        __syncthreads();
+        {
+            float a[4];
+            for (int r = 0; r < 4; r++) a[r] = L.b1[o];
+#pragma unroll 8
+            for (int i = 0; i < NIN; i++) {
+                const float w = L.w1[i * NH + o];
+                for (int r = 0; r < 4; r++) a[r] += L.x[i][s0 + r] * w;
+            }
+            for (int r = 0; r < 4; r++) gelu_both(a[r], L.h1[o][s0 + r], L.d1[o][s0 + r]);
+        }
+        __syncthreads();
+        {
+            float a[4];
+            for (int r = 0; r < 4; r++) a[r] = L.b2[o];
+#pragma unroll 8
+            for (int i = 0; i < NH; i++) {
+                const float w = L.w2[i * LW2S + o];
+                for (int r = 0; r < 4; r++) a[r] += L.h1[i][s0 + r] * w;
+            }
+            for (int r = 0; r < 4; r++) gelu_both(a[r], L.h2[o][s0 + r], L.d2[o][s0 + r]);
+        }
+        __syncthreads();
+        if (tid < TS * NOUT) {
+            const int s = tid / NOUT, c = tid % NOUT;
+            float a = L.b3[c];
+#pragma unroll 8
+            for (int i = 0; i < NH; i++) a += L.h2[i][s] * L.w3[i * NOUT + c];
+            const bool on = base + s < n;
+            if (y && on) y[(long long)(base + s) * NOUT + c] = a;
+            const float r = T && on ? a - L.t[c][s] : 0.0f;
+            L.g3[c][s] = r / rows;
+            lsum += 0.5f * r * r / rows;
+        }
+        __syncthreads();
+        if (!part) continue;
+        // layer 3: weight and input gradients
+        for (int m = 0; m < 2; m++) {
+            const int e = tid + 256 * m, i = e / NOUT, c = e % NOUT;
+            for (int s = 0; s < TS; s++) gw3[m] += L.h2[i][s] * L.g3[c][s];
+        }
+        {
+            float a[4] = {};
+#pragma unroll
+            for (int c = 0; c < NOUT; c++)
+                for (int r = 0; r < 4; r++) a[r] += L.g3[c][s0 + r] * L.w3[o * NOUT + c];
+            for (int r = 0; r < 4; r++) L.d2[o][s0 + r] *= a[r];
+        }
+        __syncthreads();
+        // layer 2
+#pragma unroll 4
+        for (int s = 0; s < TS; s++) {
+            const float g = L.d2[o][s];
+            for (int m = 0; m < NH / 4; m++) gw2[m] += L.h1[q * (NH / 4) + m][s] * g;
+        }
+        {
+            float a[4] = {};
+#pragma unroll 8
+            for (int c = 0; c < NH; c++) {
+                const float w = L.w2[o * LW2S + c];
+                for (int r = 0; r < 4; r++) a[r] += L.d2[c][s0 + r] * w;
+            }
+            for (int r = 0; r < 4; r++) L.d1[o][s0 + r] *= a[r];
+        }
+        __syncthreads();
+        // layer 1, and the biases: b1 (q = 0), b2 (q = 1), b3 (q = 2, o < 8)
+#pragma unroll 4
+        for (int s = 0; s < TS; s++) {
+            const float g = L.d1[o][s];
+            for (int m = 0; m < NIN / 4; m++) gw1[m] += L.x[q * (NIN / 4) + m][s] * g;
+        }
+        if (q < 2 || (q == 2 && o < NOUT)) {
+            const float* d = q == 0 ? L.d1[o] : (q == 1 ? L.d2[o] : L.g3[o]);
+            for (int s = 0; s < TS; s++) gb += d[s];
+        }
+    }
+    if (lpart) {
+        if (tid < TS * NOUT) L.loss[tid] = lsum;
+        __syncthreads();
+        for (int w = TS * NOUT / 2; w > 0; w >>= 1) {
+            if (tid < w) L.loss[tid] += L.loss[tid + w];
+            __syncthreads();
+        }
+        if (tid == 0) lpart[blockIdx.x] = L.loss[0];
+    }
+    if (!part) return;
+    float* P = part + (long long)blockIdx.x * NPARAM;
+    for (int m = 0; m < NIN / 4; m++) P[OFF_W1 + (q * (NIN / 4) + m) * NH + o] = gw1[m];
+    for (int m = 0; m < NH / 4; m++) P[OFF_W2 + (q * (NH / 4) + m) * NH + o] = gw2[m];
+    for (int m = 0; m < 2; m++) P[OFF_W3 + tid + 256 * m] = gw3[m];
+    if (q == 0) P[OFF_B1 + o] = gb;
+    if (q == 1) P[OFF_B2 + o] = gb;
+    if (q == 2 && o < NOUT) P[OFF_B3 + o] = gb;
+}
+
+// gradient = sum of the blocks' (64 parameters per block, a sixteenth of the
+// blocks per wave), and with lr > 0 the Adam update (Kingma and Ba 2015) with
+// the bias-corrected step size; block 0 adds the blocks' losses in float64
+constexpr int RW = 16;
+__global__ __launch_bounds__(64 * RW) void k_reduce(const float* __restrict__ part, const float* __restrict__ lpart,
+                                                    int nblk, float* __restrict__ gr, float* __restrict__ loss,
+                                                    float* __restrict__ th, float* __restrict__ m,
+                                                    float* __restrict__ v, float lr, float b1, float b2, float eps,
+                                                    float c1, float c2)
+{
+    __shared__ float red[RW][64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int t = blockIdx.x * 64 + lane;
+    float a = 0.0f;
+    if (t < NPARAM)
+#pragma unroll 4
+        for (int b = w; b < nblk; b += RW) a += part[(long long)b * NPARAM + t];
+    red[w][lane] = a;
+    __syncthreads();
+    if (w == 0 && t < NPARAM) {
+        float g = red[0][lane];
+        for (int r = 1; r < RW; r++) g += red[r][lane];
+        gr[t] = g;
+        if (lr > 0.0f) {
+            float mm = b1 * m[t] + (1.0f - b1) * g;
+            float vv = b2 * v[t] + (1.0f - b2) * g * g;
+            m[t] = mm;
+            v[t] = vv;
+            th[t] -= lr * (mm / c1) / (sqrtf(vv / c2) + eps);
+        }
+    }
+    if (blockIdx.x == 0 && w == 1) {
+        double l = 0.0;
+        for (int b = lane; b < nblk; b += 64) l += (double)lpart[b];
+        for (int off = 32; off > 0; off >>= 1) l += __shfl_xor(l, off, 64);
+        if (lane == 0) *loss = (float)l;
+    }
 }
 
 // D = A B for A[i][k] = (i + 2k mod 7) / 8, B[k][j] = (3k + j mod 5) / 4 - 0.5
@@ -151,14 +255,15 @@ struct dmx_mlp {
     float* gr = nullptr;     // gradient
     float* m = nullptr;
     float* v = nullptr;
-    float* ws = nullptr;     // per-batch workspace
+    float* ws = nullptr;     // workspace
     float* X = nullptr;      // resident data set
     float* T = nullptr;
     long long ndata = 0;
     long long adam_t = 0;
     hipStream_t stream = nullptr;
-    // workspace views
-    float *xb, *tb, *a1, *h1, *a2, *h2, *y, *g3, *g2, *g1, *part;
+    // workspace views: a batch from the host and its outputs, the blocks'
+    // gradients and losses, the losses of up to LCAP steps
+    float *xb, *tb, *y, *part, *lpart, *loss;
 };
 
 #define MCHK(x)                                                                           \
@@ -171,57 +276,22 @@ struct dmx_mlp {
     } while (0)
 
 static int cdivi(long long a, int b) { return (int)((a + b - 1) / b); }
+constexpr int LCAP = 4096;
 
-// forward of n <= cap rows already in m->xb; leaves a1, h1, a2, h2, y
-static int fwd(dmx_mlp* m, int n)
+static int blocks_of(int n) { return std::min(MAXBLK, cdivi(n, TS)); }
+
+// loss and gradient of n rows (X, T, ndata, key as k_fwd_bwd), the loss left
+// in *loss on the device; with lr > 0 an Adam step
+static int gradient(dmx_mlp* m, const float* X, const float* T, long long ndata, int n, unsigned long long key,
+                    float* loss, float lr, float b1, float b2, float eps, float c1, float c2)
 {
-    const float* W1 = m->th + OFF_W1; const float* b1 = m->th + OFF_B1;
-    const float* W2 = m->th + OFF_W2; const float* b2 = m->th + OFF_B2;
-    const float* W3 = m->th + OFF_W3; const float* b3 = m->th + OFF_B3;
-    hipLaunchKernelGGL(k_dense_fwd, dim3(cdivi((long long)n * NH, 256)), dim3(256), 0, m->stream, m->xb, NIN, W1, b1,
-                       NH, n, m->a1, m->h1);
-    hipLaunchKernelGGL(k_dense_fwd, dim3(cdivi((long long)n * NH, 256)), dim3(256), 0, m->stream, m->h1, NH, W2, b2,
-                       NH, n, m->a2, m->h2);
-    hipLaunchKernelGGL(k_dense_fwd, dim3(cdivi((long long)n * NOUT, 256)), dim3(256), 0, m->stream, m->h2, NH, W3,
-                       b3, NOUT, n, m->y, (float*)nullptr);
+    const int nb = blocks_of(n);
+    hipLaunchKernelGGL(k_fwd_bwd, dim3(nb), dim3(256), 0, m->stream, X, T, ndata, n, key, (const float*)m->th,
+                       (float*)nullptr, m->part, m->lpart);
+    hipLaunchKernelGGL(k_reduce, dim3(cdivi(NPARAM, 64)), dim3(64 * RW), 0, m->stream, (const float*)m->part,
+                       (const float*)m->lpart, nb, m->gr, loss, m->th, m->m, m->v, lr, b1, b2, eps, c1, c2);
     MCHK(hipGetLastError());
     return DMX_OK;
-}
-
-// loss and gradient of the rows in xb/tb (after fwd); loss stays on device
-static int bwd(dmx_mlp* m, int n)
-{
-    const float* W2 = m->th + OFF_W2;
-    const float* W3 = m->th + OFF_W3;
-    int nb = cdivi((long long)n * NOUT, 256);
-    hipLaunchKernelGGL(k_out_grad, dim3(nb), dim3(256), 0, m->stream, m->y, m->tb, n, m->g3, m->part);
-    hipLaunchKernelGGL(k_dense_wgrad, dim3(NOUT), dim3(256), 0, m->stream, m->h2, NH, m->g3, NOUT, n,
-                       m->gr + OFF_W3, m->gr + OFF_B3);
-    hipLaunchKernelGGL(k_dense_igrad, dim3(cdivi((long long)n * NH, 256)), dim3(256), 0, m->stream, m->g3, NOUT, W3,
-                       NH, n, m->a2, m->g2);
-    hipLaunchKernelGGL(k_dense_wgrad, dim3(NH), dim3(256), 0, m->stream, m->h1, NH, m->g2, NH, n, m->gr + OFF_W2,
-                       m->gr + OFF_B2);
-    hipLaunchKernelGGL(k_dense_igrad, dim3(cdivi((long long)n * NH, 256)), dim3(256), 0, m->stream, m->g2, NH, W2,
-                       NH, n, m->a1, m->g1);
-    hipLaunchKernelGGL(k_dense_wgrad, dim3(NH), dim3(256), 0, m->stream, m->xb, NIN, m->g1, NH, n, m->gr + OFF_W1,
-                       m->gr + OFF_B1);
-    MCHK(hipGetLastError());
-    return DMX_OK;
-}
-
-static float sum_parts(dmx_mlp* m, int nparts, int* rc)
-{
-    std::vector<float> h(nparts);
-    if (hipMemcpyAsync(h.data(), m->part, sizeof(float) * nparts, hipMemcpyDeviceToHost, m->stream) != hipSuccess ||
-        hipStreamSynchronize(m->stream) != hipSuccess) {
-        dmx::set_error("loss readback failed");
-        *rc = DMX_E_HIP;
-        return 0.0f;
-    }
-    double s = 0.0;
-    for (float x : h) s += x;
-    *rc = DMX_OK;
-    return (float)s;
 }
 
 extern "C" {
@@ -236,7 +306,7 @@ int dmx_mlp_create(int32_t max_batch, dmx_mlp** out)
     dmx_mlp* m = new dmx_mlp();
     m->cap = max_batch;
     size_t cap = (size_t)max_batch;
-    size_t wsz = cap * (NIN + NOUT + 4 * NH + NOUT + NOUT + 2 * NH) + cdivi((long long)cap * NOUT, 256) + 64;
+    size_t wsz = cap * (NIN + NOUT + NOUT) + (size_t)MAXBLK * (NPARAM + 1) + LCAP;
     if (hipStreamCreate(&m->stream) != hipSuccess || hipMalloc(&m->th, sizeof(float) * NPARAM) != hipSuccess ||
         hipMalloc(&m->gr, sizeof(float) * NPARAM) != hipSuccess || hipMalloc(&m->m, sizeof(float) * NPARAM) != hipSuccess ||
         hipMalloc(&m->v, sizeof(float) * NPARAM) != hipSuccess || hipMalloc(&m->ws, sizeof(float) * wsz) != hipSuccess) {
@@ -247,15 +317,10 @@ int dmx_mlp_create(int32_t max_batch, dmx_mlp** out)
     float* p = m->ws;
     m->xb = p; p += cap * NIN;
     m->tb = p; p += cap * NOUT;
-    m->a1 = p; p += cap * NH;
-    m->h1 = p; p += cap * NH;
-    m->a2 = p; p += cap * NH;
-    m->h2 = p; p += cap * NH;
     m->y = p; p += cap * NOUT;
-    m->g3 = p; p += cap * NOUT;
-    m->g2 = p; p += cap * NH;
-    m->g1 = p; p += cap * NH;
-    m->part = p;
+    m->part = p; p += (size_t)MAXBLK * NPARAM;
+    m->lpart = p; p += MAXBLK;
+    m->loss = p;
     hipMemsetAsync(m->th, 0, sizeof(float) * NPARAM, m->stream);
     hipMemsetAsync(m->m, 0, sizeof(float) * NPARAM, m->stream);
     hipMemsetAsync(m->v, 0, sizeof(float) * NPARAM, m->stream);
@@ -301,8 +366,10 @@ int dmx_mlp_forward(dmx_mlp* m, const float* X, int32_t n, float* Y)
 {
     if (!m || !X || !Y || n < 1 || n > m->cap) { dmx::set_error("dmx_mlp_forward: bad arguments"); return DMX_E_PARAM; }
     MCHK(hipMemcpyAsync(m->xb, X, sizeof(float) * (size_t)n * NIN, hipMemcpyHostToDevice, m->stream));
-    int rc = fwd(m, n);
-    if (rc) return rc;
+    hipLaunchKernelGGL(k_fwd_bwd, dim3(blocks_of(n)), dim3(256), 0, m->stream, (const float*)m->xb,
+                       (const float*)nullptr, 0LL, n, 0ULL, (const float*)m->th, m->y, (float*)nullptr,
+                       (float*)nullptr);
+    MCHK(hipGetLastError());
     MCHK(hipMemcpyAsync(Y, m->y, sizeof(float) * (size_t)n * NOUT, hipMemcpyDeviceToHost, m->stream));
     MCHK(hipStreamSynchronize(m->stream));
     return DMX_OK;
@@ -316,11 +383,10 @@ int dmx_mlp_loss_grad(dmx_mlp* m, const float* X, const float* T, int32_t n, flo
     }
     MCHK(hipMemcpyAsync(m->xb, X, sizeof(float) * (size_t)n * NIN, hipMemcpyHostToDevice, m->stream));
     MCHK(hipMemcpyAsync(m->tb, T, sizeof(float) * (size_t)n * NOUT, hipMemcpyHostToDevice, m->stream));
-    int rc = fwd(m, n);
-    if (!rc) rc = bwd(m, n);
+    int rc = gradient(m, m->xb, m->tb, 0, n, 0, m->loss, 0.0f, 0.0f, 0.0f, 0.0f, 1.0f, 1.0f);
     if (rc) return rc;
-    *loss = sum_parts(m, cdivi((long long)n * NOUT, 256), &rc);
-    if (rc) return rc;
+    MCHK(hipMemcpyAsync(loss, m->loss, sizeof(float), hipMemcpyDeviceToHost, m->stream));
+    MCHK(hipStreamSynchronize(m->stream));
     MCHK(hipMemcpy(grad, m->gr, sizeof(float) * NPARAM, hipMemcpyDeviceToHost));
     return DMX_OK;
 }
@@ -351,22 +417,19 @@ int dmx_mlp_train(dmx_mlp* m, int32_t steps, int32_t batch, float lr, uint64_t s
     }
     if (!m->ndata) { dmx::set_error("dmx_mlp_train: no data loaded"); return DMX_E_STATE; }
     const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
-    const int nparts = cdivi((long long)batch * NOUT, 256);
-    for (int s = 0; s < steps; s++) {
-        unsigned long long key = seed * 0x632be59bd9b4e019ULL + (unsigned long long)(m->adam_t + 1) * 0x9e3779b97f4a7c15ULL;
-        hipLaunchKernelGGL(k_gather, dim3(cdivi(batch, 256)), dim3(256), 0, m->stream, (const float*)m->X,
-                           (const float*)m->T, m->ndata, batch, key, m->xb, m->tb);
-        int rc = fwd(m, batch);
-        if (!rc) rc = bwd(m, batch);
-        if (rc) return rc;
-        m->adam_t++;
-        float c1 = 1.0f - powf(b1, (float)m->adam_t), c2 = 1.0f - powf(b2, (float)m->adam_t);
-        hipLaunchKernelGGL(k_adam, dim3(cdivi(NPARAM, 256)), dim3(256), 0, m->stream, m->th, (const float*)m->gr, m->m,
-                           m->v, NPARAM, lr, b1, b2, eps, c1, c2);
-        MCHK(hipGetLastError());
-        if (losses) {
-            losses[s] = sum_parts(m, nparts, &rc);
+    for (int s0 = 0; s0 < steps; s0 += LCAP) {
+        const int ns = std::min(LCAP, steps - s0);
+        for (int s = 0; s < ns; s++) {
+            unsigned long long key = seed * 0x632be59bd9b4e019ULL + (unsigned long long)(m->adam_t + 1) * 0x9e3779b97f4a7c15ULL;
+            m->adam_t++;
+            float c1 = 1.0f - powf(b1, (float)m->adam_t), c2 = 1.0f - powf(b2, (float)m->adam_t);
+            int rc = gradient(m, m->X, m->T, m->ndata, batch, key, m->loss + s, lr, b1, b2, eps, c1, c2);
             if (rc) return rc;
+        }
+        if (losses) {
+            // the losses of these steps, read back once
+            MCHK(hipMemcpyAsync(losses + s0, m->loss, sizeof(float) * ns, hipMemcpyDeviceToHost, m->stream));
+            MCHK(hipStreamSynchronize(m->stream));
         }
     }
     MCHK(hipStreamSynchronize(m->stream));
