@@ -2,6 +2,7 @@
 // so every kernel reproduces the reference bit for bit.
 #define DMX_T double
 #define DMX_NS f64
+#define DMX_LANE_DIR 1
 #include "dmx_step.inc"
 
 #include <mutex>

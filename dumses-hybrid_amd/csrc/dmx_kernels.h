@@ -34,6 +34,10 @@
 #ifndef DMX_BOTH_FACES
 #define DMX_BOTH_FACES 0
 #endif
+// 1: the fused kernel's threads hold one direction each (dmx_fused.inc)
+#ifndef DMX_LANE_DIR
+#define DMX_LANE_DIR 0
+#endif
 
 namespace dmx {
 

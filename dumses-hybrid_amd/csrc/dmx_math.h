@@ -45,6 +45,21 @@ __device__ __forceinline__ T tvd_slope(T qm1, T q0, T qp1, int st)
     return dsgn * fmn(dlim, fab(dcen));
 }
 
+// float64, 16 instructions instead of 20: st half / st is one factor (an exact
+// scaling, st being 1 or 2), the lesser one-sided difference a hardware
+// minimum, and the sign is copied (a NaN still comes through dcen)
+template <>
+__device__ __forceinline__ double tvd_slope<double>(double qm1, double q0, double qp1, int st)
+{
+    const double s = double(st), c = st == 1 ? 0.5 : 0.25;
+    double dlft = s * (q0 - qm1);
+    double drgt = s * (qp1 - q0);
+    double dcen = c * (dlft + drgt);
+    double dlim = __builtin_fmin(fab(dlft), fab(drgt));
+    if ((dlft * drgt) <= 0.0) dlim = 0.0;
+    return copysign(fmn(dlim, fab(dcen)), dcen);
+}
+
 // fast magnetosonic speed, the expression shared by comp_speed
 // (physics.f90:148-164) and the Riemann solvers (solver.f90:675-683):
 // b2 is passed already summed in the caller's order
