@@ -1,0 +1,37 @@
+"""Kernels that cut a domain into columns of their own: the FARGO advection
+(256 consecutive cells a block) and the shearing ghosts (64 rows a block),
+against the oracle bit for bit at the edges of their tiles."""
+import numpy as np
+import pytest
+
+import oracle as O
+from dmx import abi
+from dmx import problems as P
+
+pytestmark = pytest.mark.gpu
+
+
+def _same(pb, p, steps):
+    o = O.Oracle(p, pb.uin)
+    t_o, dts_o = o.advance(steps)
+    d = abi.Domain(p, pb.uin)
+    t_g, dts_g = d.advance(steps, 0.0)
+    assert t_o == t_g and np.array_equal(dts_o, dts_g)
+    inner = (slice(None, 8), slice(3, -3), slice(3, -3), slice(3, -3))
+    got, want = d.download(), o.store()
+    assert np.array_equal(got[inner], want[inner]), float(np.abs(got - want)[inner].max())
+    d.close()
+
+
+# rows shorter and longer than the box's shift, one block and a ragged second
+# one, ny on both sides of 64, every slope type the remap knows
+SHEAR = [dict(n=(4, 64, 5)), dict(n=(5, 65, 4), slope_type=1), dict(n=(63, 4, 3), slope_type=0),
+         dict(n=(250, 3, 3)), dict(n=(7, 130, 3), omega0=3.0)]
+
+
+@pytest.mark.parametrize("case", range(len(SHEAR)))
+def test_shearing_box_columns(case):
+    kw = dict(SHEAR[case])
+    pb = P.shearing_box(*kw.pop("n"), **kw)
+    print(f"[gpu] shearing box columns, case {case}", flush=True)
+    _same(pb, pb.params, 3)
