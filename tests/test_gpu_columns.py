@@ -1,6 +1,7 @@
 """Kernels that cut a domain into columns of their own: the FARGO advection
 (256 consecutive cells a block) and the shearing ghosts (64 rows a block),
-against the oracle bit for bit at the edges of their tiles."""
+against the oracle bit for bit at the edges of their tiles; and a state carried
+through the transfers, which stage it where the trace summary lies."""
 import numpy as np
 import pytest
 
@@ -35,3 +36,24 @@ def test_shearing_box_columns(case):
     pb = P.shearing_box(*kw.pop("n"), **kw)
     print(f"[gpu] shearing box columns, case {case}", flush=True)
     _same(pb, pb.params, 3)
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+def test_transfers_leave_the_run_unchanged(precision):
+    """Downloads between steps change nothing, and an upload of a download
+    goes on as the run does (its right faces are not read)."""
+    pb = P.random_smooth(21, 6, 9, seed=77, precision=precision)
+    print(f"[gpu] transfers, precision {precision}", flush=True)
+    a, b = abi.Domain(pb.params, pb.uin), abi.Domain(pb.params, pb.uin)
+    a.advance(1, 0.0)
+    mid = a.download()
+    a.advance(1)
+    want = a.download()
+    assert np.array_equal(want, a.download())
+    mid[8:] = np.nan
+    b.upload(mid)
+    b.time = 0.0
+    b.advance(1)
+    assert np.array_equal(b.download(), want)
+    for d in (a, b):
+        d.close()
