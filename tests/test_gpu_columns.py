@@ -1,7 +1,8 @@
 """Kernels that cut a domain into columns of their own: the FARGO advection
-(256 consecutive cells a block) and the shearing ghosts (64 rows a block),
-against the oracle bit for bit at the edges of their tiles; and a state carried
-through the transfers, which stage it where the trace summary lies."""
+(256 consecutive cells a block), the shearing ghosts (64 rows a block) and the
+viscous fluxes (tiles of at most 33 x 16 columns, 2 to 8 planes), against the
+oracle bit for bit at the edges of their tiles; and a state carried through
+the transfers, which stage it where the trace summary lies."""
 import numpy as np
 import pytest
 
@@ -36,6 +37,20 @@ def test_shearing_box_columns(case):
     pb = P.shearing_box(*kw.pop("n"), **kw)
     print(f"[gpu] shearing box columns, case {case}", flush=True)
     _same(pb, pb.params, 3)
+
+
+# one tile of 33 columns, one of 34 (two of 17), 32 x 8, narrow tiles of 16
+# rows, and planes that leave a short last block
+VISC = [(32, 6, 5), (33, 7, 4), (31, 8, 9), (4, 33, 17), (65, 5, 3)]
+
+
+@pytest.mark.parametrize("case", range(len(VISC)))
+def test_viscous_tiles(case):
+    pb = P.random_smooth(*VISC[case], seed=300 + case)
+    p = pb.params.replace(nu=2e-3, eta=1e-3 if case % 2 else 0.0, iso=1 if case == 3 else 0,
+                          ciso=1.0 if case == 3 else pb.params.ciso)
+    print(f"[gpu] viscous tiles, case {case}", flush=True)
+    _same(pb, p, 3)
 
 
 @pytest.mark.parametrize("precision", [0, 1])
