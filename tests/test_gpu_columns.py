@@ -1,8 +1,9 @@
 """Kernels that cut a domain into columns of their own: the FARGO advection
 (256 consecutive cells a block), the shearing ghosts (64 rows a block) and the
 viscous fluxes (tiles of at most 33 x 16 columns, 2 to 8 planes), against the
-oracle bit for bit at the edges of their tiles; and a state carried through
-the transfers, which stage it where the trace summary lies."""
+oracle bit for bit at the edges of their tiles; the launch shapes of a context
+as created; and a state carried through the transfers, which stage it where the
+trace summary lies."""
 import numpy as np
 import pytest
 
@@ -51,6 +52,25 @@ def test_viscous_tiles(case):
                           ciso=1.0 if case == 3 else pb.params.ciso)
     print(f"[gpu] viscous tiles, case {case}", flush=True)
     _same(pb, p, 3)
+
+
+# float64 launch shapes as created: one plane block under and over the line
+# from which the fused kernel is taken (51 tiles of 17 x 5; 10 and 11 blocks of
+# 4 planes), and tiles of which too few columns are used
+@pytest.mark.parametrize("n", [(50, 84, 40), (50, 84, 43), (34, 100, 60), (84, 84, 172)])
+def test_default_shape_gives_the_separate_kernels_bits(n):
+    pb = P.random_smooth(*n, seed=sum(n))
+    print(f"[gpu] default launch shape {n}", flush=True)
+    a, b, c = (abi.Domain(pb.params, pb.uin) for _ in range(3))
+    b.set_shape((0, 2), (0, 4))
+    a.advance(2, 0.0)
+    b.advance(2, 0.0)
+    want = b.download()
+    assert np.array_equal(a.download(), want)
+    abi.Batch([c]).advance(2)   # keeps the separate kernels
+    assert np.array_equal(c.download(), want)
+    for d in (a, b, c):
+        d.close()
 
 
 @pytest.mark.parametrize("precision", [0, 1])
