@@ -42,17 +42,17 @@ ALG_BYTES_PER_ZONE_CYCLE = {"f64": 128, "f32": 96}
 # bytes per interior cell of each kernel group's own staging, its inputs
 # read once and its outputs written once (8-byte words in float64; T-size
 # words for the bulk in float32, face B and E always float64).  The trace
-# summary has 47 words per cell, the face fluxes 18, the edge EMFs 3.  This
+# summary has 38 words per cell, the face fluxes 18, the edge EMFs 3.  This
 # is this design's intermediate traffic, not algorithmic work: reported as
 # stage_bytes_per_cell beside the roofline.
 def stage_bytes(group: str, wt: int, wb: int = 8) -> float:
     state = 4 * wt + 4 * wb
     table = {
         "compute_dt": state,
-        "trace": state + 47 * wt,
-        "faces": 47 * wt + 18 * wt,
-        "edges": 47 * wt + 3 * wt,
-        "flux": 47 * wt + 18 * wt + 3 * wt,           # faces and edges in one pass
+        "trace": state + 38 * wt,
+        "faces": 38 * wt + 18 * wt,
+        "edges": 38 * wt + 3 * wt,
+        "flux": 38 * wt + 18 * wt + 3 * wt,           # faces and edges in one pass
         "fused": state + 18 * wt + 3 * wt,            # trace + faces + edges in one pass
         "update_ct": 2 * state + 18 * wt + 3 * wt,
         # learned limiter: state -> 8 float primitives -> 24 float slopes
@@ -69,25 +69,22 @@ def stage_bytes(group: str, wt: int, wb: int = 8) -> float:
 # the launch shapes the autotuner keeps at 256^3.  Constants copied from
 # that file; COUNTERS_SOURCE names the file and the commit whose kernels it
 # measured.
-COUNTERS_SOURCE = ("profiles/mhd_step_ot256_hbm_bytes.md, profiles/mhd_step_ot256_sq_counters.md, "
-                   "profiles/fused_trace_flux_ot256.md (kernel code of commit 0f60dc7; the files name the launch shapes)")
+COUNTERS_SOURCE = ("profiles/mhd_step_ot256_hbm_bytes.md, profiles/mhd_step_ot256_sq_counters.md "
+                   "(kernel code of commit d048f04; the files name the launch shapes)")
 MEASURED_TRAFFIC = {
-    "f64": {"trace": 570.6, "flux": 1876.8, "update_ct": 414.4, "compute_dt": 86.3,
-            "boundary": 17.7},
-    "f32": {"fused": 234.5, "update_ct": 295.0, "compute_dt": 69.5, "boundary": 14.8},
+    "f64": {"fused": 464.0, "update_ct": 415.9, "compute_dt": 85.8, "boundary": 17.7},
+    "f32": {"fused": 234.6, "update_ct": 295.1, "compute_dt": 69.5, "boundary": 14.8},
 }
 
 
 # VALU-busy fraction of each kernel group at 256^3 (SQ_ACTIVE_INST_VALU x 4
 # / 1024 SIMDs / kernel cycles) from the rocprofv3 SQ counter runs summarised
-# in profiles/mhd_step_ot256_sq_counters.md and profiles/fused_trace_flux_ot256.md:
+# in profiles/mhd_step_ot256_sq_counters.md:
 # the bound that applies where the HBM fraction is low (bit-exact float64
 # division and square root)
 MEASURED_VALU_BUSY = {
-    "f64": {"trace": 0.504, "flux": 0.702, "update_ct": 0.371, "compute_dt": 0.730, "boundary": 0.049,
-            "fused": 0.502},
-    "f32": {"trace": 0.413, "flux": 0.640, "update_ct": 0.232, "compute_dt": 0.401, "boundary": 0.057,
-            "fused": 0.608},
+    "f64": {"fused": 0.605, "update_ct": 0.336, "compute_dt": 0.734, "boundary": 0.048},
+    "f32": {"fused": 0.615, "update_ct": 0.227, "compute_dt": 0.391, "boundary": 0.057},
 }
 
 
@@ -121,7 +118,7 @@ def roofline(prof: dict, cells: int, prec: str) -> dict | None:
 # planes), (trace mode, planes)); --no-tune applies them without timing, so
 # that profiler runs measure the kernels of the timed run (under a profiler
 # the autotuner's timings, and so its choice, can change)
-TUNED_256 = {0: ((0, 2), (1, 16)), 1: ((3, 16), (1, 32))}
+TUNED_256 = {0: ((3, 16), (1, 16)), 1: ((3, 16), (1, 32))}
 # --fused: the trace and the face/edge stage in one kernel (mode 3, the trace
 # summary kept in LDS), 16 planes per block, in place of the tuned pair
 FUSED_SHAPE = ((3, 16), (1, 16))
