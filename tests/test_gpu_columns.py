@@ -73,6 +73,34 @@ def test_default_shape_gives_the_separate_kernels_bits(n):
         d.close()
 
 
+# the forms that the default takes to the fused kernel: solvers, limiters,
+# boundaries, isothermal, shear with and without FARGO, dissipation
+FORMS = [dict(riemann=P.HLL, riemann2d=P.LLF, slope_type=1), dict(riemann=P.LLF, riemann2d=P.UPWIND, slope_type=3),
+         dict(riemann=P.UPWIND, riemann2d=P.HLLA, slope_type=0), dict(iso=1, ciso=1.0),
+         dict(bdtype=(P.ZERO_GRADIENT, P.ZERO_GRADIENT, P.PERIODIC)), dict(nu=1e-3, eta=1e-3),
+         dict(shear=0), dict(shear=1), dict(shear=0, iso=1, ciso=4e-2)]
+
+
+@pytest.mark.parametrize("form", range(len(FORMS)))
+def test_default_fused_form_gives_the_separate_kernels_bits(form):
+    kw = dict(FORMS[form])
+    n = (50, 84, 43)
+    if "shear" in kw:
+        pb = P.shearing_box(*n, fargo=kw.pop("shear"))
+    else:
+        pb = P.random_smooth(*n, seed=form)
+    p = pb.params.replace(**kw)
+    print(f"[gpu] default fused form {form}", flush=True)
+    a, b = abi.Domain(p, pb.uin), abi.Domain(p, pb.uin)
+    b.set_shape((0, 2), (0, 4))
+    _, da = a.advance(2, 0.0)
+    _, db = b.advance(2, 0.0)
+    assert np.isfinite(da).all() and np.array_equal(da, db)
+    assert np.array_equal(a.download(), b.download())
+    for d in (a, b):
+        d.close()
+
+
 @pytest.mark.parametrize("precision", [0, 1])
 def test_transfers_leave_the_run_unchanged(precision):
     """Downloads between steps change nothing, and an upload of a download
