@@ -9,6 +9,7 @@ import pytest
 
 import oracle as O
 from dmx import abi
+from dmx import learned
 from dmx import problems as P
 
 pytestmark = pytest.mark.gpu
@@ -74,11 +75,12 @@ def test_default_shape_gives_the_separate_kernels_bits(n):
 
 
 # the forms that the default takes to the fused kernel: solvers, limiters,
-# boundaries, isothermal, shear with and without FARGO, dissipation
+# boundaries, isothermal, shear with and without FARGO, dissipation, the learned
+# limiter
 FORMS = [dict(riemann=P.HLL, riemann2d=P.LLF, slope_type=1), dict(riemann=P.LLF, riemann2d=P.UPWIND, slope_type=3),
          dict(riemann=P.UPWIND, riemann2d=P.HLLA, slope_type=0), dict(iso=1, ciso=1.0),
          dict(bdtype=(P.ZERO_GRADIENT, P.ZERO_GRADIENT, P.PERIODIC)), dict(nu=1e-3, eta=1e-3),
-         dict(shear=0), dict(shear=1), dict(shear=0, iso=1, ciso=4e-2)]
+         dict(shear=0), dict(shear=1), dict(shear=0, iso=1, ciso=4e-2), dict(slope_type=4)]
 
 
 @pytest.mark.parametrize("form", range(len(FORMS)))
@@ -93,6 +95,9 @@ def test_default_fused_form_gives_the_separate_kernels_bits(form):
     print(f"[gpu] default fused form {form}", flush=True)
     a, b = abi.Domain(p, pb.uin), abi.Domain(p, pb.uin)
     b.set_shape((0, 2), (0, 4))
+    if p.slope_type == 4:
+        for d in (a, b):
+            d.set_limiter(learned.init_params(5))
     _, da = a.advance(2, 0.0)
     _, db = b.advance(2, 0.0)
     assert np.isfinite(da).all() and np.array_equal(da, db)
