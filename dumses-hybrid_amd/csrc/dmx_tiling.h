@@ -1,7 +1,8 @@
 // dmx_tiling.h -- how the z-marching kernels cut a domain into column
 // tiles and blocks of planes.  Plain integer code for host and device;
 // tests/tiling_check.cpp compiles it on the host and checks that the tiles
-// cover every column and plane exactly once within their limits.
+// cover every column and plane exactly once within their limits,
+// tests/launch_check.cpp the limits of the launches.
 #pragma once
 
 #ifndef __HIPCC__
@@ -80,6 +81,16 @@ __host__ __device__ __forceinline__ void tiling_tile(const Tiling& t, int l, int
     }
     part_tile(t.px, xt, x0, fx);
     part_tile(t.pz, zb, z0, fz);
+}
+
+// Whether the face/edge stage over one plane per block, a grid of x * y * z
+// blocks, may be launched as one block per Riemann problem of a cell: at most
+// `most` blocks (kSplitMax in dmx_step.inc), and 6 z blocks along z, which
+// counts planes times problems, within the 65535 that a grid has along y and z
+// (float32 domains of nx <= 60 and ny = 3 reach 6 x 16384 otherwise).
+inline bool split_fits(long long x, long long y, long long z, long long most)
+{
+    return x * y * z <= most && 6 * z <= 65535;
 }
 
 } // namespace dmx
