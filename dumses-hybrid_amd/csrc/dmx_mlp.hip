@@ -49,17 +49,18 @@ struct TrainLds {
     float h1[NH][TS], d1[NH][TS];                // gelu(a1), gelu'(a1); then d1 holds dL/da1
     float h2[NH][TS], d2[NH][TS];
     float g3[NOUT][TS];                          // dL/dy
-    float loss[TS * NOUT];
+    double loss[TS * NOUT];
     long long row[TS];
 };
 
 // X, T: data (rows drawn by the hash of key when ndata > 0, else row s of the
 // batch is row s); n rows in the batch; y: outputs (may be null); part: block
-// gradients (null: forward only); lpart: block sums of 0.5 (y - T)^2 / n
+// gradients (null: forward only); lpart: block sums of 0.5 (y - T)^2 / n, in
+// float64 from the single terms on
 __global__ __launch_bounds__(256) void k_fwd_bwd(const float* __restrict__ X, const float* __restrict__ T, long long ndata,
                                                  int n, unsigned long long key, const float* __restrict__ th,
                                                  float* __restrict__ y, float* __restrict__ part,
-                                                 float* __restrict__ lpart)
+                                                 double* __restrict__ lpart)
 {
     __shared__ TrainLds L;
     const int tid = threadIdx.x;
@@ -74,7 +75,8 @@ __global__ __launch_bounds__(256) void k_fwd_bwd(const float* __restrict__ X, co
     // thread (o, q): column o of a layer, rows 4 q .. 4 q + 3 of the tile (and
     // quarter q of a weight matrix's rows)
     const int o = tid & 63, q = tid >> 6, s0 = 4 * q;
-    float gw1[NIN / 4] = {}, gw2[NH / 4] = {}, gw3[2] = {}, gb = 0.0f, lsum = 0.0f;
+    float gw1[NIN / 4] = {}, gw2[NH / 4] = {}, gw3[2] = {}, gb = 0.0f;
+    double lsum = 0.0;   // float64: a block of a large batch adds hundreds of tiles' terms
     const float rows = (float)n;
     const int ntile = (n + TS - 1) / TS;
     for (int tile = blockIdx.x; tile < ntile; tile += gridDim.x) {
@@ -193,7 +195,7 @@ __global__ __launch_bounds__(256) void k_fwd_bwd(const float* __restrict__ X, co
 // blocks per wave), and with lr > 0 the Adam update (Kingma and Ba 2015) with
 // the bias-corrected step size; block 0 adds the blocks' losses in float64
 constexpr int RW = 16;
-__global__ __launch_bounds__(64 * RW) void k_reduce(const float* __restrict__ part, const float* __restrict__ lpart,
+__global__ __launch_bounds__(64 * RW) void k_reduce(const float* __restrict__ part, const double* __restrict__ lpart,
                                                     int nblk, float* __restrict__ gr, float* __restrict__ loss,
                                                     float* __restrict__ th, float* __restrict__ m,
                                                     float* __restrict__ v, float lr, float b1, float b2, float eps,
@@ -222,7 +224,7 @@ __global__ __launch_bounds__(64 * RW) void k_reduce(const float* __restrict__ pa
     }
     if (blockIdx.x == 0 && w == 1) {
         double l = 0.0;
-        for (int b = lane; b < nblk; b += 64) l += (double)lpart[b];
+        for (int b = lane; b < nblk; b += 64) l += lpart[b];
         for (int off = 32; off > 0; off >>= 1) l += __shfl_xor(l, off, 64);
         if (lane == 0) *loss = (float)l;
     }
@@ -263,7 +265,8 @@ struct dmx_mlp {
     hipStream_t stream = nullptr;
     // workspace views: a batch from the host and its outputs, the blocks'
     // gradients and losses, the losses of up to LCAP steps
-    float *xb, *tb, *y, *part, *lpart, *loss;
+    float *xb, *tb, *y, *part, *loss;
+    double* lpart;
 };
 
 #define MCHK(x)                                                                           \
@@ -289,7 +292,7 @@ static int gradient(dmx_mlp* m, const float* X, const float* T, long long ndata,
     hipLaunchKernelGGL(k_fwd_bwd, dim3(nb), dim3(256), 0, m->stream, X, T, ndata, n, key, (const float*)m->th,
                        (float*)nullptr, m->part, m->lpart);
     hipLaunchKernelGGL(k_reduce, dim3(cdivi(NPARAM, 64)), dim3(64 * RW), 0, m->stream, (const float*)m->part,
-                       (const float*)m->lpart, nb, m->gr, loss, m->th, m->m, m->v, lr, b1, b2, eps, c1, c2);
+                       (const double*)m->lpart, nb, m->gr, loss, m->th, m->m, m->v, lr, b1, b2, eps, c1, c2);
     MCHK(hipGetLastError());
     return DMX_OK;
 }
@@ -306,7 +309,7 @@ int dmx_mlp_create(int32_t max_batch, dmx_mlp** out)
     dmx_mlp* m = new dmx_mlp();
     m->cap = max_batch;
     size_t cap = (size_t)max_batch;
-    size_t wsz = cap * (NIN + NOUT + NOUT) + (size_t)MAXBLK * (NPARAM + 1) + LCAP;
+    size_t wsz = cap * (NIN + NOUT + NOUT) + (size_t)MAXBLK * (NPARAM + 2) + LCAP;
     if (hipStreamCreate(&m->stream) != hipSuccess || hipMalloc(&m->th, sizeof(float) * NPARAM) != hipSuccess ||
         hipMalloc(&m->gr, sizeof(float) * NPARAM) != hipSuccess || hipMalloc(&m->m, sizeof(float) * NPARAM) != hipSuccess ||
         hipMalloc(&m->v, sizeof(float) * NPARAM) != hipSuccess || hipMalloc(&m->ws, sizeof(float) * wsz) != hipSuccess) {
@@ -319,7 +322,8 @@ int dmx_mlp_create(int32_t max_batch, dmx_mlp** out)
     m->tb = p; p += cap * NOUT;
     m->y = p; p += cap * NOUT;
     m->part = p; p += (size_t)MAXBLK * NPARAM;
-    m->lpart = p; p += MAXBLK;
+    static_assert((NIN + NOUT + NOUT) % 2 == 0 && NPARAM % 2 == 0, "float64 alignment of lpart");
+    m->lpart = (double*)p; p += 2 * MAXBLK;
     m->loss = p;
     hipMemsetAsync(m->th, 0, sizeof(float) * NPARAM, m->stream);
     hipMemsetAsync(m->m, 0, sizeof(float) * NPARAM, m->stream);
@@ -368,7 +372,7 @@ int dmx_mlp_forward(dmx_mlp* m, const float* X, int32_t n, float* Y)
     MCHK(hipMemcpyAsync(m->xb, X, sizeof(float) * (size_t)n * NIN, hipMemcpyHostToDevice, m->stream));
     hipLaunchKernelGGL(k_fwd_bwd, dim3(blocks_of(n)), dim3(256), 0, m->stream, (const float*)m->xb,
                        (const float*)nullptr, 0LL, n, 0ULL, (const float*)m->th, m->y, (float*)nullptr,
-                       (float*)nullptr);
+                       (double*)nullptr);
     MCHK(hipGetLastError());
     MCHK(hipMemcpyAsync(Y, m->y, sizeof(float) * (size_t)n * NOUT, hipMemcpyDeviceToHost, m->stream));
     MCHK(hipStreamSynchronize(m->stream));
