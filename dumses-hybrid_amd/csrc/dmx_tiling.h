@@ -2,7 +2,7 @@
 // tiles and blocks of planes.  Plain integer code for host and device;
 // tests/tiling_check.cpp compiles it on the host and checks that the tiles
 // cover every column and plane exactly once within their limits,
-// tests/launch_check.cpp the limits of the launches.
+// tests/launch_check.cpp the limits and choices of the launches.
 #pragma once
 
 #ifndef __HIPCC__
@@ -91,6 +91,37 @@ __host__ __device__ __forceinline__ void tiling_tile(const Tiling& t, int l, int
 inline bool split_fits(long long x, long long y, long long z, long long most)
 {
     return x * y * z <= most && 6 * z <= 65535;
+}
+
+// Planes per block of the fused float64 kernel where it is not tuned: 16 where
+// that gives 768 blocks (1.5 rounds of the 512 that the chip holds), else 4.
+inline int fused_planes(int nx, int ny, int nz, int fxm, int fym, int fc)
+{
+    const Tiling t = make_tiling(nx + 1, ny + 1, nz + 1, fxm, fym, fc, 16);
+    return (long long)t.tz * t.pz.nt >= 768 ? 16 : 4;
+}
+
+// Whether the fused float64 kernel over the tiles t is the faster form of the
+// trace and the face/edge stage, by what the two take (us).  Fused: a block
+// marches its planes and the one before them, 512 blocks (two per CU) at a time,
+// 12.5 us a plane for each round begun, or 13.5 for a full one and 6 for the
+// end of the last where the rounds run into one another.  Separate: 36 ns a
+// block of 64 x 4 columns of a plane and 0.283 ns a cell.  So thin boxes and
+// few blocks, which pay the extra plane and a second round that is nearly
+// empty, keep the separate kernels.  Over 67 domains of 3 to 1000 cells a side
+// with HLLD, and the other solvers over 13 of them, the choice is at most
+// 5.8% from the faster one; measured (us, fused / separate): 101 x 50 x 37 133
+// / 89, 118 x 60 x 30 134 / 94, 224 x 224 x 6 197 / 149, 128 x 256 x 8 160 / 139,
+// 48^3 91 / 67, but 64^3 144 / 161, 512 x 512 x 8 940 / 1011, 80 x 48 x 243 418 /
+// 517, 150 x 93 x 117 655 / 722 and 192^3 2617 / 3135.
+inline bool fused_pays(const Tiling& t, int nx, int ny, int nz)
+{
+    const long long blocks = (long long)t.tz * t.pz.nt, begun = (blocks + 511) / 512;
+    const double drift = 13.5 * (double)blocks / 512.0 + 6.0;
+    const double fused = ((double)(nz + 1) / t.pz.nt + 1.0) * (12.5 * begun > drift ? 12.5 * begun : drift);
+    const double nb = (double)((nx + 4 + 63) / 64) * ((ny + 1 + 3) / 4) * (nz + 1);
+    const double separate = 4.0 + 0.036 * nb + 0.283e-3 * (nx + 1) * (ny + 1) * (nz + 1);
+    return fused < separate;
 }
 
 } // namespace dmx

@@ -1,7 +1,9 @@
 // Host check of launch limits (dumses-hybrid_amd/csrc/dmx_tiling.h): over the
 // thin and long domains that dmx_create accepts, a face/edge stage launched as
 // one block per Riemann problem stays within 65535 blocks along z, whatever its
-// line in blocks.  Prints "bad 0" on success.
+// line in blocks; and over domains measured on an MI355X in float64, the kernel
+// that fused_pays takes is at most 6% slower than the other.  Prints "bad 0" on
+// success.
 #include <cstdio>
 #include <initializer_list>
 
@@ -24,6 +26,32 @@ int main()
                     if (!s && 6 * z <= 65535 && x * y * z <= most) bad++;
                     s ? split++ : whole++;
                 }
+    // us of the trace and the face/edge stage (HLLD, MC): fused over
+    // fused_planes, and the separate kernels as created
+    const struct { int nx, ny, nz; double fused, separate; } seen[] = {
+        {224, 224, 3, 120.8, 98}, {224, 224, 6, 196.6, 148.7}, {224, 224, 12, 302.1, 273.9},
+        {224, 224, 16, 373.5, 384.6}, {224, 224, 24, 540, 562.3}, {512, 512, 3, 448.5, 467.1},
+        {512, 512, 8, 940.4, 1011.2}, {128, 256, 8, 160.4, 139}, {700, 101, 4, 172.5, 155.2},
+        {300, 300, 5, 255.1, 226.4}, {300, 300, 12, 509.8, 508.5}, {64, 64, 64, 143.7, 160.9},
+        {96, 96, 96, 401.5, 430.4}, {128, 128, 128, 869.4, 962.7}, {33, 300, 20, 133.3, 115.8},
+        {50, 84, 43, 119.1, 94.4}, {67, 67, 67, 147.5, 173.4}, {101, 50, 37, 132.9, 88.9},
+        {16, 400, 40, 136.3, 207.7}, {400, 16, 40, 161, 114.5}, {272, 90, 9, 141.2, 107.1},
+        {118, 60, 30, 133.6, 93.8}, {80, 80, 26, 89.1, 94.3}, {39, 24, 98, 92.5, 61.6}, {52, 160, 23, 143.9, 98.9},
+        {30, 92, 225, 300.4, 395.6}, {80, 48, 243, 418.3, 516.8}, {156, 26, 81, 176.5, 139.5},
+        {95, 45, 74, 177.1, 151.6}, {79, 69, 184, 515.2, 557.1}, {279, 349, 7, 325.6, 339.4},
+        {266, 591, 11, 746, 810.6}, {192, 192, 192, 2616.6, 3134.5}, {150, 93, 117, 654.6, 721.6},
+        {32, 64, 32, 69.5, 52.7}, {48, 48, 48, 91, 67.2},
+    };
+    for (const auto& m : seen) {
+        const Tiling t = make_tiling(m.nx + 1, m.ny + 1, m.nz + 1, 17, 5, 85,
+                                     fused_planes(m.nx, m.ny, m.nz, 17, 5, 85));
+        const double got = fused_pays(t, m.nx, m.ny, m.nz) ? m.fused : m.separate;
+        const double best = m.fused < m.separate ? m.fused : m.separate;
+        if (got > 1.06 * best) {
+            if (bad++ < 20)
+                printf("bad choice: n %d %d %d: %.1f us, the other %.1f\n", m.nx, m.ny, m.nz, got, best);
+        }
+    }
     printf("split %ld whole %ld bad %ld\n", split, whole, bad);
     return bad != 0 || !split || !whole;
 }
