@@ -124,4 +124,32 @@ inline bool fused_pays(const Tiling& t, int nx, int ny, int nz)
     return fused < separate;
 }
 
+// A batch's launch shapes from context 0's: face/edge stage (mode 0 or 2 over
+// 4 << kzi planes, 3 over 8 << kzi), trace (mode, z-march over 8 << kti planes).
+// Shapes that were asked for (by the tuner, dmx_set_shape or the environment)
+// are taken over, or the nearest that a batch has: 1 and 2 planes are 4, the
+// separate face and edge kernels mode 0.  A context's own shapes are made for
+// one box: a batch fills the chip with the separate kernels over 4 planes and
+// the 3D tile of the trace.  Measured (ms a step, float64 / float32): 6 boxes of
+// 128^3 6.7 / 3.61, over 8 planes 6.8 / 3.64, with the z-march of the trace 7.1 /
+// 3.94, fused in float64 10.2; 16 of 64^3 2.64 / 1.49, 2.82 / 1.52, 2.76 / 1.59,
+// 3.8; 48 of 32^3 1.30 / 0.70, 1.33 / 0.73, 1.37 / 0.78.  4 float64 boxes of
+// 150 x 93 x 117, whose own trace is the z-march, take 3.36 with the tile, 3.47
+// with the z-march.
+struct BatchShape { int flux_mode, kzi, trace_mode, kti; };
+inline BatchShape batch_shape(int flux_mode, int kz, bool flux_asked, int trace_mode, int kt, bool trace_asked)
+{
+    auto near = [](int k) { return k <= 11 ? 0 : (k <= 23 ? 1 : 2); };   // of 8, 16, 32
+    BatchShape b = {0, 0, 0, 1};
+    if (flux_asked) {
+        b.flux_mode = flux_mode == 1 ? 0 : flux_mode;
+        b.kzi = flux_mode == 3 ? near(kz) : (kz <= 4 ? 0 : (kz == 16 ? 2 : (kz == 32 ? 3 : 1)));
+    }
+    if (trace_asked) {
+        b.trace_mode = trace_mode;
+        b.kti = near(kt);
+    }
+    return b;
+}
+
 } // namespace dmx

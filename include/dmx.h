@@ -234,9 +234,11 @@ int  dmx_batch_advance(dmx_batch* batch, int32_t nsteps, double* times);
  * kernel, 4/8/16/32 planes per block) after that trace against the trace
  * and face/edge stage in one kernel (mode 3, 8/16/32 planes); state
  * unchanged; best_ms is the chosen stage kernel's time, shape[4] as
- * dmx_tune.  A batch starts with context 0's shapes (a z-march or mode 3
- * over another plane count takes the nearest of 8, 16, 32; face/edge mode
- * 1 takes mode 0). */
+ * dmx_tune.  A batch starts with the shapes that context 0 was given by
+ * dmx_tune or dmx_set_shape (a z-march or mode 3 over another plane count
+ * takes the nearest of 8, 16, 32; face/edge mode 1 takes mode 0, 1 and 2
+ * planes 4); if it was given none, with the separate kernels: the 16x4x4 tile
+ * of the trace, the face/edge stage over 4 planes. */
 int  dmx_batch_tune(dmx_batch* batch, double* best_ms, int32_t* shape);
 /* milliseconds of the last dmx_batch_advance on the device */
 int  dmx_batch_last_ms(dmx_batch* batch, double* ms);

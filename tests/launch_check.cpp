@@ -52,6 +52,26 @@ int main()
                 printf("bad choice: n %d %d %d: %.1f us, the other %.1f\n", m.nx, m.ny, m.nz, got, best);
         }
     }
+    // context 0's {flux mode, planes, asked, trace mode, planes, asked} and the
+    // batch's {flux mode, kzi, trace mode, kti}
+    const struct { int fm, kz; bool fa; int tm, kt; bool ta; BatchShape want; } shapes[] = {
+        {0, 1, false, 0, 16, false, {0, 0, 0, 1}}, {0, 2, false, 1, 16, false, {0, 0, 0, 1}},
+        {3, 16, false, 1, 32, false, {0, 0, 0, 1}}, {3, 16, true, 1, 32, true, {3, 1, 1, 2}},
+        {3, 4, true, 0, 16, true, {3, 0, 0, 1}}, {3, 32, true, 1, 8, true, {3, 2, 1, 0}},
+        {1, 8, true, 1, 11, true, {0, 1, 1, 0}}, {0, 1, true, 1, 12, true, {0, 0, 1, 1}},
+        {0, 2, true, 0, 16, true, {0, 0, 0, 1}}, {0, 4, true, 1, 64, true, {0, 0, 1, 2}},
+        {2, 16, true, 0, 16, false, {2, 2, 0, 1}}, {2, 32, true, 1, 16, false, {2, 3, 0, 1}},
+        {0, 8, true, 1, 16, false, {0, 1, 0, 1}}, {3, 16, false, 1, 16, true, {0, 0, 1, 1}},
+    };
+    for (const auto& q : shapes) {
+        const BatchShape b = batch_shape(q.fm, q.kz, q.fa, q.tm, q.kt, q.ta);
+        if (b.flux_mode != q.want.flux_mode || b.kzi != q.want.kzi || b.trace_mode != q.want.trace_mode
+            || b.kti != q.want.kti) {
+            if (bad++ < 20)
+                printf("bad batch shape of {%d %d %d, %d %d %d}: {%d %d %d %d}\n", q.fm, q.kz, q.fa, q.tm, q.kt, q.ta,
+                       b.flux_mode, b.kzi, b.trace_mode, b.kti);
+        }
+    }
     printf("split %ld whole %ld bad %ld\n", split, whole, bad);
     return bad != 0 || !split || !whole;
 }
