@@ -124,6 +124,30 @@ inline bool fused_pays(const Tiling& t, int nx, int ny, int nz)
     return fused < separate;
 }
 
+// Planes per block (4, 8, 16 or 32) with which the fused float32 kernel, one
+// block per CU, marches the fewest planes one after another: rounds of 256
+// blocks times the planes of a block and the one before them, the fewer planes
+// if it is the same within 1%.  A round takes 9.0 to 9.7 us a plane at any size
+// from 96^3 on, so this is the fastest count or within 2% of it: 4, 8, 16, 32
+// planes measured 216, 188, 167, 302 us at 96^3, 332, 355, 321, 354 at 112^3, 440, 442, 474, 602
+// at 128^3, 782, 739, 785, 902 at 160^3, 1346, 1285, 1274, 1234 at 192^3 and
+// 3080, 2857, 2717, 2764 at 256^3.
+inline int fewest_plane_rounds(int nx, int ny, int nz, int fxm, int fym, int fc)
+{
+    int pick = 4;
+    double least = 0.0;
+    for (int kt = 4; kt <= 32; kt *= 2) {
+        const Tiling t = make_tiling(nx + 1, ny + 1, nz + 1, fxm, fym, fc, kt);
+        const long long rounds = ((long long)t.tz * t.pz.nt + 255) / 256;
+        const double planes = (double)rounds * ((double)(nz + 1) / t.pz.nt + 1.0);
+        if (kt == 4 || planes < 0.99 * least) {
+            least = planes;
+            pick = kt;
+        }
+    }
+    return pick;
+}
+
 // A batch's launch shapes from context 0's: face/edge stage (mode 0 or 2 over
 // 4 << kzi planes, 3 over 8 << kzi), trace (mode, z-march over 8 << kti planes).
 // Shapes that were asked for (by the tuner, dmx_set_shape or the environment)

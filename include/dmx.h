@@ -195,6 +195,10 @@ const char* dmx_kernel_name(int32_t id);
  * the face/edge stage's time per launch (mode 3: trace included) in
  * *best_ms and {face/edge mode, planes, trace mode, planes} in shape[4]
  * (either may be NULL).  Every shape gives the same results in float64.
+ * In float32 the last bits differ between shapes, and the learned limiter
+ * amplifies them (its mode 3 takes the planes from the sizes, without
+ * timing): a float32 run that is to be repeated bit for bit sets its shape
+ * with dmx_set_shape.
  * The state is unchanged.  No counterpart in the reference's step: it takes
  * the role of utils/pyutils/gpuconfig/gpuconfig.py, which sweeps OpenACC
  * vector sizes by re-running the code. */

@@ -1,9 +1,11 @@
-// Host check of launch limits (dumses-hybrid_amd/csrc/dmx_tiling.h): over the
-// thin and long domains that dmx_create accepts, a face/edge stage launched as
-// one block per Riemann problem stays within 65535 blocks along z, whatever its
-// line in blocks; and over domains measured on an MI355X in float64, the kernel
-// that fused_pays takes is at most 6% slower than the other.  Prints "bad 0" on
-// success.
+// Host check of the launch limits and choices of
+// dumses-hybrid_amd/csrc/dmx_tiling.h: over the thin and long domains that
+// dmx_create accepts, a face/edge stage launched as one block per Riemann problem
+// stays within 65535 blocks along z, whatever its line in blocks; over domains
+// measured on an MI355X, the kernel that fused_pays takes in float64 is at most
+// 6% slower than the other, and the planes of the learned limiter's fused kernel
+// at most 2% slower than the fastest; a batch takes over the shapes asked for,
+// not those a context was created with.  Prints "bad 0" on success.
 #include <cstdio>
 #include <initializer_list>
 
@@ -71,6 +73,25 @@ int main()
                 printf("bad batch shape of {%d %d %d, %d %d %d}: {%d %d %d %d}\n", q.fm, q.kz, q.fa, q.tm, q.kt, q.ta,
                        b.flux_mode, b.kzi, b.trace_mode, b.kti);
         }
+    }
+    // us of the fused float32 kernel with the learned limiter over 4, 8, 16 and
+    // 32 planes per block, measured: the count by the sizes is at most 2% slower
+    // than the fastest
+    const struct { int nx, ny, nz; double us[4]; } marched[] = {
+        {32, 32, 32, {58.6, 91.2, 161.5, 301.1}},         {48, 48, 48, {59.5, 91.8, 160.9, 440.6}},
+        {64, 64, 64, {63.0, 94.1, 161.7, 302.2}},         {80, 80, 80, {160.0, 183.6, 162.5, 369.3}},
+        {96, 96, 96, {216.0, 187.8, 167.3, 301.6}},       {112, 112, 112, {331.6, 355.2, 321.4, 354.3}},
+        {128, 128, 128, {440.1, 442.1, 474.4, 602.1}},    {160, 160, 160, {781.8, 738.5, 785.3, 901.8}},
+        {192, 192, 192, {1346.2, 1285.0, 1274.3, 1233.6}}, {256, 256, 256, {3080.2, 2856.7, 2717.4, 2764.4}},
+        {100, 60, 77, {114.3, 173.2, 189.0, 353.2}},      {33, 100, 51, {95.0, 93.5, 168.8, 462.7}},
+        {128, 32, 64, {110.7, 92.2, 160.3, 298.8}},
+    };
+    for (const auto& m : marched) {
+        const int kt = fewest_plane_rounds(m.nx, m.ny, m.nz, 33, 8, 256);
+        const double got = m.us[kt == 4 ? 0 : kt == 8 ? 1 : kt == 16 ? 2 : 3];
+        for (double us : m.us)
+            if (got > 1.02 * us && bad++ < 20)
+                printf("bad planes: n %d %d %d: %d planes, %.1f us against %.1f\n", m.nx, m.ny, m.nz, kt, got, us);
     }
     printf("split %ld whole %ld bad %ld\n", split, whole, bad);
     return bad != 0 || !split || !whole;
