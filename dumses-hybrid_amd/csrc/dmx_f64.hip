@@ -107,20 +107,13 @@ int compute_dt_noalloc(const dmx_params& p, const double* uin, double* dt, hipSt
     HIPCHK(scratch_ptr(dev, &part));
     Step st;
     memset(&st, 0, sizeof(st));
-    Geom& g = st.g;
-    g.nx = p.nx; g.ny = p.ny; g.nz = p.nz;
-    g.dx = (p.xmax - p.xmin) / p.nx;
-    g.dy = (p.ymax - p.ymin) / p.ny;
-    g.dz = (p.zmax - p.zmin) / p.nz;
-    g.xmin = p.xmin; g.xmax = p.xmax; g.ymin = p.ymin; g.ymax = p.ymax; g.zmin = p.zmin; g.zmax = p.zmax;
-    st.ph.gamma = p.gamma; st.ph.ciso = p.ciso; st.ph.omega0 = p.omega0; st.ph.courant = p.courant;
-    st.ph.iso = p.iso; st.ph.fargo = p.fargo;
+    set_step(st, p);
     const long long ncell = (long long)p.nx * p.ny * p.nz;
     const long long want = (ncell + 255) / 256;
     const int nb = (int)(want < kNoAllocPartials ? want : kNoAllocPartials);
     hipLaunchKernelGGL(k_dt_uin_min, dim3(nb), dim3(256), 0, stream, st, uin, part);
     hipLaunchKernelGGL(k_dt_uin_final, dim3(1), dim3(256), 0, stream, (const double*)part, nb,
-                       p.courant * g.dx / 1e-10, p.courant, dt);
+                       p.courant * st.g.dx / 1e-10, p.courant, dt);
     HIPCHK(hipGetLastError());
     return DMX_OK;
 }
