@@ -120,7 +120,8 @@ def roofline(prof: dict, cells: int, prec: str) -> dict | None:
 # the autotuner's timings, and so its choice, can change)
 TUNED_256 = {0: ((3, 16), (1, 16)), 1: ((3, 16), (1, 32))}
 # --fused: the trace and the face/edge stage in one kernel (mode 3, the trace
-# summary kept in LDS), 16 planes per block, in place of the tuned pair
+# summary kept in LDS), 16 planes per block, without timing other shapes; at 256^3
+# that is what the autotuner keeps too
 FUSED_SHAPE = ((3, 16), (1, 16))
 
 
@@ -280,7 +281,7 @@ def main():
                     help="apply the launch shapes the autotuner keeps at 256^3 instead of tuning")
     ap.add_argument("--fused", action="store_true",
                     help="run the trace and the face/edge stage as one kernel (launch mode 3) "
-                         "instead of the tuned pair")
+                         "over 16 planes, instead of tuning")
     ap.add_argument("--calibrate", action="store_true",
                     help="also run a plain 1 GiB device copy (torch) to calibrate HBM byte counters")
     a = ap.parse_args()
